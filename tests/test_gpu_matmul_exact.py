@@ -1,6 +1,6 @@
-"""matmul_t on the exact-integer fp16 kernel (aq_matmul_h.hip: Q4_K weights as
-sc*code integers, Q6_K weights as q - 32 with d*sc per 16-element group in
-fp32, on fp16 matrix cores, X in two fp16 pieces after a per-row
+"""matmul_t on the exact-integer fp16 kernels (aq_matmul_h.hip,
+aq_matmul_hd.hip: Q4_K weights as sc*code integers, Q6_K weights as sc*(q - 32)
+in two exact halves, on fp16 matrix cores, X in two fp16 pieces after a per-row
 power-of-two scale, d and dmin applied in fp32) against the float64 oracle
 (oracle/qmatrix_ref.py, the reference's QuantMatrix.matmul_t,
 alpacca/qmatrix.py:184-211).  Bar: 2e-5 normalized by ||W_r|| * ||x_m||, the
@@ -448,3 +448,43 @@ def test_exact_fp16_fused_x_unsplit_is_m_invariant(dtype):
     parts = np.concatenate([qm.matmul_t(X[a:b], precision="fp32")
                             for a, b in ((0, 7), (7, 23), (23, 39), (39, 150))])
     assert np.array_equal(whole.view(np.uint32), parts.view(np.uint32))
+
+
+# Tile kernel (aq_matmul_hd.hip): every shape at sizes that end inside a tile
+# of each, with the split lengths 1 group and several.  Bar: 2^-22 of
+# ||W_r|| ||x_m|| from the two pieces of x, and as much again for the fp32
+# sums (at most 24 chained products per group and cols / 256 groups).
+TILE_TOL = 2.0 ** -21
+
+
+@pytest.mark.parametrize("dtype", ["Q4_K", "Q5_K", "Q6_K", "Q8_0", "Q4_0", "Q4_1", "Q5_0", "Q5_1"])
+@pytest.mark.parametrize("M,rows,cols", [(1, 1, 256), (17, 129, 512), (129, 385, 768)])
+def test_tile_shapes_vs_f64(dtype, M, rows, cols, monkeypatch):
+    """Each shape against float64, and the same bits from all of them at fp32
+    (no split of K); AUTO may split."""
+    data = synth.random_matrix_bytes(dtype, rows, cols, seed=rows + cols)
+    X = synth.random_x(cols, seed=M, batch=M)
+    qm = QuantMatrix(data, dtype, rows, cols)
+    want, norms = _f64(data, rows, cols, X, dtype)
+    first = None
+    for shape in range(5):
+        monkeypatch.setenv("AQ_MATMUL_TILE", str(shape))
+        Y = qm.matmul_t(X, precision="fp32")
+        assert normalized_error(Y, want, norms, X) < TILE_TOL, shape
+        if first is None:
+            first = Y
+        assert np.array_equal(Y.view(np.uint32), first.view(np.uint32)), shape
+        if M > 16:
+            assert normalized_error(qm.matmul_t(X), want, norms, X) < TILE_TOL, shape
+
+
+@pytest.mark.parametrize("layout", ["raw", "split"])
+@pytest.mark.parametrize("dtype", ["Q4_K", "Q5_K"])
+def test_tile_kernel_layouts_agree(dtype, layout):
+    """The DMA takes a super-block's fields from either layout's planes."""
+    M, rows, cols = 70, 200, 2304
+    data = synth.random_matrix_bytes(dtype, rows, cols, seed=31)
+    X = synth.random_x(cols, seed=32, batch=M)
+    want, norms = _f64(data, rows, cols, X, dtype)
+    Y = QuantMatrix(data, dtype, rows, cols, layout=layout).matmul_t(X)
+    assert normalized_error(Y, want, norms, X) < TILE_TOL
