@@ -866,181 +866,299 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// The same batched causal attention on fp32 matrix cores
-// (v_mfma_f32_16x16x4f32), the default form: the fp32 products and sums of
-// the VALU kernel above at twice its speed (552 -> 268 us per layer of the
-// 1B model's 2048-token prefill).  The grid, the rows of a wave (16 (token, head)
-// rows, 16 / G tokens times the G heads) and the online softmax over
-// 64-position chunks are k_attn_prefill's.  Per chunk, staged in LDS (K
-// row-major, V transposed):
+// The same batched causal attention on bf16 matrix cores with every fp32
+// operand in three bf16 pieces (24 bits), the default form.  x = x0 + x1 + x2
+// with x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1); a product x y is
+// the six piece products of index sum at most 2, smallest first, in one fp32
+// accumulator (what is dropped is below 2^-25 of it), so products and sums
+// keep fp32's accuracy at 6/16 of the fp32 matrix cores' time
+// (v_mfma_f32_16x16x32_bf16 against 16x16x4f32).  No scaling is needed: bf16
+// has fp32's exponent range.  A non-finite q, K or V makes the rows that see it
+// non-finite.
+//
+// Grid: one workgroup of NW waves per (16 NW (token, head) rows, kv head); a
+// wave owns 16 rows (16 / G tokens times the G heads) and keeps the online
+// softmax of k_attn_prefill over 64-position chunks.  Per chunk the workgroup cuts K and V into pieces in LDS (K row-major, V
+// transposed, 16-byte chunks swizzled by row), then per wave:
 //   S^T (positions x rows) = K Q^T: lane l holds row l % 16's scores at
 //     positions 16 pt + 4 (l / 16) + r (four 16-position tiles pt, r = 0..3);
-//     the k index of lane group c = l / 16 in step s is dimension c HD/4 + s,
-//     so a lane's q fragment and K reads are HD/4 consecutive floats;
-//   the row's maximum and sum over the chunk: the lane's 16 scores, then the
-//     four lanes of the row (xor 16, xor 32);
-//   O^T (dimensions x rows) += V^T P^T: the weights are the B operand as the
-//     lanes hold them (step (pt, r) takes position 16 pt + 4 c + r in lane
-//     group c), V^T the A operand, so the rescale of O by e^(m - m') is a
-//     lane's own row.
-// The output is O / l.  Positions past a token's own are masked.
+//   the row's maximum over the chunk: the lane's 16 scores, then the four
+//     lanes of the row; the row's sum stays per lane until the end;
+//   O^T (dimensions x rows) += V^T P^T: a lane's weights of two position
+//     tiles are its B operand as it holds them (lane group g: positions 32 u +
+//     4 g .. +3 and 32 u + 16 + 4 g .. +3; V^T's columns are stored in that
+//     order).  The weights' pieces are cut by truncation (exact).
+//
+// 32 / 8 heads of 64, 2048 tokens (a 1B layer): 257 us on fp32 matrix cores,
+// 119 here; of 128, 609 -> 205; 100 tokens at position 1000 62 -> 44 and 128 ->
+// 76; error against float64 4.0e-7 -> 2.9e-7 and 4.5e-7 -> 3.0e-7.  What bounds
+// it: per wave and chunk of 64 dimensions 96 matrix products (1,536 cycles)
+// and about as many cycles of VALU (softmax and the pieces of the weights, 800;
+// the pieces of the wave's share of the chunk, 700), on three waves per SIMD.
+// Two row tiles per wave (half the pieces' work, 216 registers) measured 128
+// us, eight waves on one chunk 146.
+typedef __bf16 bf16x8_ __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4_ __attribute__((ext_vector_type(4)));
+typedef float f4v_ __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint32_t pack_bf16_(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+// the three pieces of (a, b), packed
+__device__ __forceinline__ void pieces3(float a, float b, uint32_t (&o)[3]) {
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    o[p] = pack_bf16_(a, b);
+    a -= __uint_as_float(o[p] << 16);
+    b -= __uint_as_float(o[p] & 0xFFFF0000u);
+  }
+}
+// the same by truncation: exact, 8 bits a piece
+__device__ __forceinline__ void pieces3_cut(float a, float b, uint32_t (&o)[3]) {
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    o[p] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+    a -= __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
+    b -= __uint_as_float(__float_as_uint(b) & 0xFFFF0000u);
+  }
+}
 template <int HD, int G, int NW>
 __global__ void __launch_bounds__(64 * NW)
     k_attn_prefill_mfma(const float *__restrict__ q, const float *__restrict__ kc,
                         const float *__restrict__ vc, const aq_decode_state *st, int64_t pos0,
-                        int64_t n_ctx, int64_t T, float scale, float *__restrict__ out) {
-  constexpr int NTG = kPfRows, TPW = NTG / G, TPB = NW * TPW, CH = 64, NT = 64 * NW;
-  constexpr int KS = HD / 4;          // k steps of S^T (dimensions per lane)
-  constexpr int NHT = HD / 16;        // 16-dimension tiles of O^T
-  constexpr int LK = HD + 4, LV = CH + 4;  // LDS row strides (floats)
-  constexpr int F4 = CH * HD / 4;     // float4 of K (and of V) per chunk
-  constexpr int PT = F4 / NT;         // per thread
-  static_assert(F4 % NT == 0 && KS % 4 == 0, "the chunk divides over the threads");
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float *Ks = lds;            // [CH][LK]
-  float *Vt = Ks + CH * LK;   // [HD][LV]
+                        int64_t n_ctx, int64_t T, float scale, int tiles, int fold,
+                        float *__restrict__ out) {
+  constexpr int TPW = kPfRows / G, TPB = NW * TPW;  // tokens per wave, block
+  constexpr int CH = 64, NT = 64 * NW;
+  constexpr int KS = HD / 32;   // k steps of S^T
+  constexpr int NHT = HD / 16;  // 16-dimension tiles of O^T
+  constexpr int D4 = HD / 4, ITEMS = 16 * D4, PT = (ITEMS + NT - 1) / NT;
+  static_assert(ITEMS % NT == 0, "the chunk divides over the threads");
+  constexpr int KP = CH * HD * 2, VP = KP;  // LDS bytes of a piece plane
+  extern __shared__ __attribute__((aligned(16))) uint8_t pfs[];
+  uint8_t *Ks = pfs, *Vs = pfs + 3 * KP;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r16 = lane & 15, cg = lane >> 4;
-  const int kvh = blockIdx.y, n_head = gridDim.y * G;
-  const int64_t tw = (int64_t)blockIdx.x * TPB + wave * TPW;  // this wave's first token
-  const int64_t pb = st ? (int64_t)st->pos : pos0;            // position of token 0
-  // this lane's row (r16): token, head, last position it may see
+  // Work grows with the token tile: the heavy tiles first, kv heads side by
+  // side (XCD = workgroup id modulo 8: a kv head's K and V stay in one L2).
+  // fold: all workgroups resident at once, two to a CU; the second half runs
+  // light to heavy so that each CU's pair adds up alike.
+  const int n_kv = gridDim.x / tiles;
+  int rank = blockIdx.x / n_kv;
+  const int kvh = blockIdx.x % n_kv, n_head = n_kv * G;
+  if (fold && rank >= (tiles + 1) / 2) rank = tiles - 1 - (rank - (tiles + 1) / 2);
+  const int tile = tiles - 1 - rank;
+  const int64_t tw = (int64_t)tile * TPB + wave * TPW;  // this wave's first token
+  const int64_t pb = st ? (int64_t)st->pos : pos0;      // position of token 0
+  // this lane's row: token and head
   const int64_t t_row = tw + r16 / G;
   const int h_row = kvh * G + r16 % G;
-  const int64_t lim = pb + t_row;
-  // q fragment: dimensions cg*KS .. cg*KS + KS - 1 of the row (zeros past T)
-  float qf[KS];
+  bf16x8_ qf[KS][3];
 #pragma unroll
-  for (int j = 0; j < KS / 4; ++j) {
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (t_row < T) v = reinterpret_cast<const float4 *>(q + (t_row * n_head + h_row) * HD + cg * KS)[j];
-    qf[4 * j] = v.x;
-    qf[4 * j + 1] = v.y;
-    qf[4 * j + 2] = v.z;
-    qf[4 * j + 3] = v.w;
+  for (int ks = 0; ks < KS; ++ks) {
+    f4v_ v[2] = {f4v_{0.f, 0.f, 0.f, 0.f}, f4v_{0.f, 0.f, 0.f, 0.f}};
+    if (t_row < T) {
+      const f4v_ *qr =
+          reinterpret_cast<const f4v_ *>(q + (t_row * n_head + h_row) * HD + 32 * ks + 8 * cg);
+      v[0] = qr[0];
+      v[1] = qr[1];
+    }
+    uint32_t w[4][3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pieces3(v[i >> 1][2 * (i & 1)], v[i >> 1][2 * (i & 1) + 1], w[i]);
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+      qf[ks][p] = __builtin_bit_cast(bf16x8_, u32x4_{w[0][p], w[1][p], w[2][p], w[3][p]});
   }
-  int64_t t_last = (int64_t)blockIdx.x * TPB + TPB - 1;
+  int64_t t_last = (int64_t)tile * TPB + TPB - 1;
   t_last = t_last < T ? t_last : T - 1;
-  const int n_c = (int)((pb + t_last + 1 + CH - 1) / CH);  // chunks the last token reaches
-  // (native 4-vectors: HIP's float4 struct kept these arrays in scratch)
-  typedef float f4v_ __attribute__((ext_vector_type(4)));
+  int64_t p_last = pb + t_last;  // the last position any row of the block sees
+  p_last = p_last < n_ctx ? p_last : n_ctx - 1;
+  const int n_c = (int)((p_last + CH) / CH);
   const f4v_ *kb = reinterpret_cast<const f4v_ *>(kc + (int64_t)kvh * n_ctx * HD);
   const f4v_ *vb = reinterpret_cast<const f4v_ *>(vc + (int64_t)kvh * n_ctx * HD);
-  // float4 i of a chunk: position i / (HD/4), dimensions 4 (i % (HD/4)) ..
-  f4v_ rk[PT], rv[PT];
-#define AQ_PF_FETCH(c)                                                          \
-  _Pragma("unroll") for (int j = 0; j < PT; ++j) {                             \
-    const int i = tid + NT * j;                                                 \
-    int64_t pg = (int64_t)(c) * CH + i / (HD / 4);                              \
-    pg = pg < n_ctx ? pg : n_ctx - 1; /* in bounds; such positions are masked */ \
-    rk[j] = kb[pg * (HD / 4) + i % (HD / 4)];                                   \
-    rv[j] = vb[pg * (HD / 4) + i % (HD / 4)];                                   \
-  }
+  // item: four positions 4 pq .. +3 at dimensions 4 d4 .. +3
+  f4v_ rk[PT][4], rv[PT][4];
+  auto fetch = [&](int c) {
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      const int i = tid + NT * j, d4 = i % D4, pq = i / D4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        int64_t pg = (int64_t)c * CH + 4 * pq + e;
+        pg = pg < p_last ? pg : p_last;  // past the block's last position: masked
+        rk[j][e] = kb[pg * D4 + d4];
+        rv[j][e] = vb[pg * D4 + d4];
+      }
+    }
+  };
+  auto stage = [&]() {
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      const int i = tid + NT * j, d4 = i % D4, pq = i / D4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {  // K: position row, dimensions 4 d4 ..
+        const int row = 4 * pq + e;
+        uint32_t a[3], b[3];
+        pieces3(rk[j][e][0], rk[j][e][1], a);
+        pieces3(rk[j][e][2], rk[j][e][3], b);
+        uint8_t *dst = Ks + row * HD * 2 + (((d4 >> 1) ^ (row & 7)) * 16) + 8 * (d4 & 1);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2 *>(dst + p * KP) = make_uint2(a[p], b[p]);
+      }
+      // V^T: dimension row, positions 4 pq .. +3, which are half a chunk of
+      // the stored order: chunk 4 u + g, u = pq / 8, g = pq % 4, half pq / 4 % 2
+      const int ck = 4 * (pq >> 3) + (pq & 3), half = (pq >> 2) & 1;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int dim = 4 * d4 + k;
+        uint32_t a[3], b[3];
+        pieces3(rv[j][0][k], rv[j][1][k], a);
+        pieces3(rv[j][2][k], rv[j][3][k], b);
+        uint8_t *dst = Vs + dim * 128 + ((ck ^ ((dim ^ (dim >> 3)) & 7)) * 16) + 8 * half;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2 *>(dst + p * VP) = make_uint2(a[p], b[p]);
+      }
+    }
+  };
   f4v_ o[NHT];
 #pragma unroll
   for (int ht = 0; ht < NHT; ++ht) o[ht] = f4v_{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;
-  AQ_PF_FETCH(0)
+  const float f = scale * 1.44269504088896341f;  // scores times f are exponents of 2
+  float mf = -INFINITY, l = 0.f;  // running maximum (times f), this lane's part of the sum
+  // the piece products, smallest first: (piece of A, piece of B)
+  constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
+  fetch(0);
   for (int c = 0; c < n_c; ++c) {
     __syncthreads();  // the previous chunk is consumed
-#pragma unroll
-    for (int j = 0; j < PT; ++j) {  // stage: K row-major, V transposed
-      const int i = tid + NT * j;
-      const int p = i / (HD / 4), d4 = i % (HD / 4);
-      *reinterpret_cast<f4v_ *>(&Ks[p * LK + 4 * d4]) = rk[j];
-      Vt[(4 * d4 + 0) * LV + p] = rv[j][0];
-      Vt[(4 * d4 + 1) * LV + p] = rv[j][1];
-      Vt[(4 * d4 + 2) * LV + p] = rv[j][2];
-      Vt[(4 * d4 + 3) * LV + p] = rv[j][3];
-    }
+    stage();
     __syncthreads();
-    if (c + 1 < n_c) {  // the next chunk's loads fly during this one
-      AQ_PF_FETCH(c + 1)
-    }
-    // scores S^T of the four 16-position tiles
+    if (c + 1 < n_c) fetch(c + 1);  // the next chunk's loads fly during this one
     f4v_ sc[4];
 #pragma unroll
     for (int pt = 0; pt < 4; ++pt) {
-      sc[pt] = f4v_{0.f, 0.f, 0.f, 0.f};
-      const float *kr = &Ks[(pt * 16 + r16) * LK + cg * KS];
+      const uint8_t *kr = Ks + (pt * 16 + r16) * HD * 2;
+      bf16x8_ kf[KS][3];
 #pragma unroll
-      for (int j = 0; j < KS / 4; ++j) {
-        const float4 kv = reinterpret_cast<const float4 *>(kr)[j];
-        sc[pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.x, qf[4 * j], sc[pt], 0, 0, 0);
-        sc[pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.y, qf[4 * j + 1], sc[pt], 0, 0, 0);
-        sc[pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.z, qf[4 * j + 2], sc[pt], 0, 0, 0);
-        sc[pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.w, qf[4 * j + 3], sc[pt], 0, 0, 0);
-      }
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          kf[ks][p] = *reinterpret_cast<const bf16x8_ *>(kr + p * KP + ((4 * ks + cg) ^ (r16 & 7)) * 16);
+      sc[pt] = f4v_{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int z = 0; z < 6; ++z)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          sc[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks][PA[z]], qf[ks][PB[z]], sc[pt], 0, 0, 0);
     }
-    // lane (r16, cg) of tile pt holds S^T[16 pt + 4 cg + r][row r16]
-    float mx = -INFINITY;
+    // lane (r16, cg) of tile pt holds S^T[16 pt + 4 cg + r][row r16]; chunks
+    // that end past the wave's first token are masked
+    if ((int64_t)c * CH + CH - 1 > pb + tw) {
+      const int64_t lim = pb + t_row - (int64_t)c * CH - 4 * cg;
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (pt * 16 + r > lim) sc[pt][r] = -INFINITY;
+    }
+    float mx = sc[0][0];
 #pragma unroll
     for (int pt = 0; pt < 4; ++pt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t pg = (int64_t)c * CH + pt * 16 + 4 * cg + r;
-        sc[pt][r] = pg <= lim ? sc[pt][r] * scale : -INFINITY;
-        mx = fmaxf(mx, sc[pt][r]);
-      }
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[pt][r]);
     mx = max_xor<16>(mx);
     mx = max_xor<32>(mx);
-    const float mn = fmaxf(m, mx);
-    const float corr = exp_shift(m, mn);
+    const float mn = fmaxf(mf, mx * f);
+    const float corr = mf == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mf - mn);
+    const float off = mn == -INFINITY ? 0.f : mn;
     float sum = 0.f;
 #pragma unroll
     for (int pt = 0; pt < 4; ++pt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float e = sc[pt][r] == -INFINITY ? 0.f : exp_w(sc[pt][r] - mn);
+        const float e = __builtin_amdgcn_exp2f(fmaf(sc[pt][r], f, -off));
         sc[pt][r] = e;
         sum += e;
       }
-    sum = add_xor<16>(sum);
-    sum = add_xor<32>(sum);
-    l = l * corr + sum;
-    m = mn;
+    l = fmaf(l, corr, sum);
+    mf = mn;
 #pragma unroll
-    for (int ht = 0; ht < NHT; ++ht) {
-      o[ht] *= corr;
+    for (int ht = 0; ht < NHT; ++ht) o[ht] *= corr;
 #pragma unroll
-      for (int pt = 0; pt < 4; ++pt) {
-        const float4 vv = *reinterpret_cast<const float4 *>(&Vt[(ht * 16 + r16) * LV + pt * 16 + 4 * cg]);
-        o[ht] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.x, sc[pt][0], o[ht], 0, 0, 0);
-        o[ht] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.y, sc[pt][1], o[ht], 0, 0, 0);
-        o[ht] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.z, sc[pt][2], o[ht], 0, 0, 0);
-        o[ht] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.w, sc[pt][3], o[ht], 0, 0, 0);
+    for (int u = 0; u < 2; ++u) {
+      bf16x8_ pf[3];
+      uint32_t w[4][3];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        pieces3_cut(sc[2 * u + (i >> 1)][2 * (i & 1)], sc[2 * u + (i >> 1)][2 * (i & 1) + 1], w[i]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        pf[p] = __builtin_bit_cast(bf16x8_, u32x4_{w[0][p], w[1][p], w[2][p], w[3][p]});
+#pragma unroll
+      for (int ht = 0; ht < NHT; ++ht) {
+        const int dim = ht * 16 + r16;
+        const uint8_t *vr = Vs + dim * 128 + ((4 * u + cg) ^ ((dim ^ (dim >> 3)) & 7)) * 16;
+        bf16x8_ vf[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) vf[p] = *reinterpret_cast<const bf16x8_ *>(vr + p * VP);
+#pragma unroll
+        for (int z = 0; z < 6; ++z)
+          o[ht] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[PA[z]], pf[PB[z]], o[ht], 0, 0, 0);
       }
     }
   }
-#undef AQ_PF_FETCH
   // lane (r16, cg) of tile ht holds O^T[16 ht + 4 cg + r][row r16]
+  float den = add_xor<16>(l);
+  den = add_xor<32>(den);
   if (t_row < T) {
-    const float inv = 1.f / l;
+    const float inv = 1.f / den;
 #pragma unroll
     for (int ht = 0; ht < NHT; ++ht)
-      reinterpret_cast<float4 *>(out + (t_row * n_head + h_row) * HD + ht * 16)[cg] =
-          make_float4(o[ht][0] * inv, o[ht][1] * inv, o[ht][2] * inv, o[ht][3] * inv);
+      reinterpret_cast<f4v_ *>(out + (t_row * n_head + h_row) * HD + ht * 16)[cg] = o[ht] * inv;
   }
+}
+
+template <int HD, int G, int NW>
+hipError_t prefill_attn_tiles(const float *q, const float *kc, const float *vc, int n_kv,
+                              int64_t n_ctx, const aq_decode_state *st, int64_t pos0, int64_t T,
+                              float scale, float *out, int cus, hipStream_t s) {
+  constexpr int TPB = NW * (kPfRows / G);
+  constexpr int lds = 6 * 64 * HD * 2;
+  const int tiles = (int)((T + TPB - 1) / TPB);
+  const int64_t wgs = (int64_t)tiles * n_kv;
+  const int fold = wgs > cus && wgs <= 2 * (int64_t)cus && 2 * lds <= 160 * 1024;
+  auto kern = k_attn_prefill_mfma<HD, G, NW>;
+  if (hipError_t e = set_dynamic_lds(reinterpret_cast<const void *>(kern), lds)) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * NW), lds, s, q, kc, vc, st, pos0, n_ctx,
+                     T, scale, tiles, fold, out);
+  return hipGetLastError();
 }
 
 template <int HD, int G>
 hipError_t prefill_attn_launch(const float *q, const float *kc, const float *vc, int n_kv,
                                int64_t n_ctx, const aq_decode_state *st, int64_t pos0,
                                int64_t T, float scale, float *out, hipStream_t s) {
+  // matrix cores (the default), or the VALU kernel when AQ_ATTN_PREFILL_VALU is set
+  if (!getenv("AQ_ATTN_PREFILL_VALU")) {
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev)) return e;
+    const int cus = device_info(dev).cus;
+#define AQ_PF(nw) \
+  prefill_attn_tiles<HD, G, nw>(q, kc, vc, n_kv, n_ctx, st, pos0, T, scale, out, cus, s)
+    // Four waves, 48 KB of LDS (three workgroups per CU), at head_dim 64.  At
+    // 128 one 96 KB workgroup fits a CU: eight waves once four-wave
+    // workgroups come in more than two rounds (32 / 8 heads, 2048 tokens 205
+    // against 278 us; 16 / 4 heads 171 against 150).
+    const int64_t wgs4 = (T + 4 * (kPfRows / G) - 1) / (4 * (kPfRows / G)) * n_kv;
+    if constexpr (HD == 128) {
+      if (wgs4 > 2 * (int64_t)cus) return AQ_PF(8);
+    }
+    return AQ_PF(4);
+#undef AQ_PF
+  }
   constexpr int TPB = 4 * (kPfRows / G);
   const dim3 grid((unsigned)((T + TPB - 1) / TPB), (unsigned)n_kv);
-  // matrix cores (the default; 4-wave workgroups: 26.6 ms for the 1B model's
-  // 2048-token prefill against 27.4 ms with 8 waves and 27.8 ms with 2), or
-  // the VALU kernel when AQ_ATTN_PREFILL_VALU is set (31.2 ms)
-  if (!getenv("AQ_ATTN_PREFILL_VALU")) {
-    const size_t lds = (size_t)(64 * (HD + 4) + HD * (64 + 4)) * sizeof(float);
-    hipError_t e =
-        set_dynamic_lds(reinterpret_cast<const void *>(k_attn_prefill_mfma<HD, G, 4>), (int)lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_attn_prefill_mfma<HD, G, 4>), grid, dim3(256), lds, s, q, kc, vc, st,
-                       pos0, n_ctx, T, scale, out);
-    return hipGetLastError();
-  }
   const size_t lds = (size_t)(2 * 64 * HD + 4 * HD * kPfRows + 4 * 64 * kPfRows) * sizeof(float);
   hipError_t e = set_dynamic_lds(reinterpret_cast<const void *>(k_attn_prefill<HD, G>), (int)lds);
   if (e != hipSuccess) return e;

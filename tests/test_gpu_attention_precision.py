@@ -8,6 +8,7 @@ against float64, the exact softmax)."""
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 import pytest
@@ -58,3 +59,41 @@ def test_attention_vs_f64_wide_scores(n_ctx, pos, q_scale, hd):
     print(f"attention n_ctx={n_ctx} pos={pos} hd={hd} q_scale={q_scale}: "
           f"max|out - f64| / max|V| = {err:.2e}", flush=True)
     assert err < 1e-5, (err, s_span)
+
+
+@pytest.mark.parametrize("hd,T,vscale,qscale", [(64, 130, 1e25, 1.0), (128, 1100, 1e-25, 6.0),
+                                                (64, 65, 1.0, 1e-20)])
+def test_attention_batch_three_pieces_vs_f64(hd, T, vscale, qscale):
+    """The batched attention cuts q, K, V and the weights into three bf16
+    pieces (24 bits, fp32's exponent range, no scaling): against float64 at
+    magnitudes far from one, and the same bits when the tokens come in several
+    calls (which at head_dim 128 run four-wave workgroups, the 1100 tokens
+    eight-wave ones).  Bar 1e-5 max|V|, as for the decode form above."""
+    n_head, n_kv, pos0 = 32, 8, 70
+    n_ctx = pos0 + T
+    rng = np.random.default_rng(hd + T)
+    q = (rng.standard_normal((T, n_head * hd)) * qscale).astype(np.float32)
+    K = rng.standard_normal((n_kv, n_ctx, hd)).astype(np.float32)
+    V = (rng.standard_normal((n_kv, n_ctx, hd)) * vscale).astype(np.float32)
+    kc, vc, qd = (torch.from_numpy(a).to("cuda") for a in (K, V, q))
+    lib = _lib.ensure_device()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+
+    def run(cuts):
+        out = torch.empty((T, n_head * hd), device="cuda")
+        for a, b in zip(cuts, cuts[1:]):
+            _lib.check(lib.aq_attention_batch(p(qd[a:b]), p(kc), p(vc), b - a, n_head, n_kv, hd,
+                                              n_ctx, None, pos0 + a, p(out[a:b]), None))
+        return out.cpu().numpy()
+
+    whole = run([0, T])
+    cut = sorted({0, 3, T // 3, T // 2 + 1, T})
+    assert np.array_equal(whole.view(np.uint32), run(cut).view(np.uint32))
+    for h in (0, 5, 31):
+        kv = h // (n_head // n_kv)
+        s = q[:, h * hd:(h + 1) * hd].astype(np.float64) @ K[kv].astype(np.float64).T / math.sqrt(hd)
+        s[np.arange(n_ctx)[None, :] > pos0 + np.arange(T)[:, None]] = -np.inf
+        w = np.exp(s - s.max(axis=1, keepdims=True))
+        want = (w / w.sum(axis=1, keepdims=True)) @ V[kv].astype(np.float64)
+        err = np.abs(whole[:, h * hd:(h + 1) * hd] - want).max() / np.abs(V).max()
+        assert err < 1e-5, (h, err)

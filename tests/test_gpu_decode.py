@@ -625,7 +625,7 @@ def test_tiny_model_batched_prefill(tiny, precision):
 @pytest.mark.parametrize("path", ["prefill", "prefill_valu", "chunked"])
 def test_attention_batch_causal(n_head, n_kv, hd, pos0, T, path, monkeypatch):
     """T > 1 runs the one-launch prefill kernel (online softmax over the
-    chunks; on fp32 matrix cores, or on the VALU with AQ_ATTN_PREFILL_VALU)
+    chunks; on matrix cores, or on the VALU with AQ_ATTN_PREFILL_VALU)
     unless AQ_ATTN_CHUNKED selects the decode kernels (partials per 64-position
     chunk, then the combine); all against the oracle."""
     if path == "chunked":
