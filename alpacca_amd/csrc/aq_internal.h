@@ -21,6 +21,7 @@ struct aq_matrix {
   uint8_t *dev;         // one hipMalloc holding every plane
   size_t dev_bytes;
   aq::Planes planes;
+  bool finite;          // dense: no infinity or NaN among the weights
 };
 
 namespace aq {
@@ -77,6 +78,15 @@ bool mm_h_supported(const aq_matrix *m);
 hipError_t launch_matmul_h(const aq_matrix *m, const float *X, int64_t M, float *Y,
                            bool m_invariant, hipStream_t s, float *ysw = nullptr,
                            bool *fused_sw = nullptr);
+
+// matmul_t of dense weights on 16-bit matrix cores at float32 accuracy
+// (aq_matmul_dn.hip), for matrices without infinities and NaNs
+// (mm_dn_supported; dense_all_finite looks through a matrix's device copy).
+// m_invariant as for launch_matmul_h.
+bool mm_dn_supported(const aq_matrix *m);
+hipError_t dense_all_finite(const aq_matrix *m, bool *finite);
+hipError_t launch_matmul_dn(const aq_matrix *m, const float *X, int64_t M, float *Y,
+                            bool m_invariant, hipStream_t s);
 
 // Device scratch memory for work on stream `s` of `device`, at least `bytes`
 // long (nullptr when it cannot be allocated).  One buffer per (device,

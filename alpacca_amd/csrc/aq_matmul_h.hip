@@ -29,6 +29,7 @@
 #include <algorithm>
 
 #include "aq_matmul_h.h"
+#include "aq_matmul_tiles.h"
 
 namespace aq {
 namespace {
@@ -424,14 +425,10 @@ __global__ void __launch_bounds__(512)
 }
 
 // ---- the choice of tiles ----------------------------------------------------------
-// Shapes of the tile kernel, with the time (us) of one 64-column stage when
-// every CU has one workgroup and when it has two (0: no second one fits
-// beside the first, or the shape is not built), and of the ends of a tile
-// (prologue, stores), by kind: Q4_K / Q5_K, Q6_K, the per-32 formats.
-struct TileCost {
-  int bm, bn;
-  float one[3], two[3], ends;
-};
+// Shapes of the tile kernel; kinds: Q4_K / Q5_K, Q6_K, the per-32 formats.  The
+// constants are a fit to 4,028 timed calls (Q4_K, Q6_K, Q8_0, Q5_0; N 512 -
+// 14336, K 2048 - 14336, M 5 - 1500, every shape with up to eight splits): the
+// call they pick is 0.5 % slower than the fastest on average, 10 % at worst.
 constexpr TileCost kTiles[] = {
     {128, 256, {1.86f, 0.f, 0.f}, {0.f, 0.f, 0.f}, 3.6f},
     {128, 128, {1.15f, 1.55f, 1.33f}, {0.f, 0.f, 0.f}, 1.2f},
@@ -440,45 +437,7 @@ constexpr TileCost kTiles[] = {
     {16, 128, {0.496f, 0.595f, 0.494f}, {0.513f, 0.92f, 0.75f}, 0.f},
 };
 constexpr int kTileShapes = sizeof(kTiles) / sizeof(kTiles[0]);
-// The shape and split of least estimated time: rounds of one or two
-// workgroups per CU (a launch on few CUs runs its stages up to 11 % faster
-// than one on all of them), the tiles' ends, and for a split the traffic of
-// the partials.  The constants are a fit to 4,028 timed calls (Q4_K, Q6_K,
-// Q8_0, Q5_0; N 512 - 14336, K 2048 - 14336, M 5 - 1500, every shape with
-// up to eight splits): the call it picks is 0.5 % slower than the fastest on
-// average, 10 % at worst.
-void choose_tile(int kind, int64_t M, int64_t N, int units, int cus, int max_splits, int &shape,
-                 int &splits) {
-  float best = 0.f;
-  shape = -1;
-  for (int t = 0; t < kTileShapes; ++t) {
-    const TileCost &c = kTiles[t];
-    if (c.one[kind] == 0.f) continue;
-    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-    for (int want = 1; want <= max_splits; ++want) {
-      if (want > 1 && (want > units / 2 || (want - 1) * tiles >= 2 * (int64_t)cus)) break;
-      const int per = (units + want - 1) / want, sp = (units + per - 1) / per;
-      if (sp != want) continue;
-      const int64_t wgs = tiles * sp;
-      const float low = 0.89f + 0.11f * std::min(1.f, (float)wgs / (float)cus);
-      float rounds;  // of a stage's time
-      if (c.two[kind] == 0.f) {
-        rounds = (float)((wgs + cus - 1) / cus) * c.one[kind] * low;
-      } else {
-        const int64_t full = wgs / (2 * cus), rest = wgs - full * 2 * cus;
-        rounds = (float)full * c.two[kind] +
-                 (rest > cus ? c.two[kind] : rest > 0 ? c.one[kind] * low : 0.f);
-      }
-      float us = rounds * 4.f * (float)per + c.ends * (float)((wgs + cus - 1) / cus);
-      if (sp > 1) us += 0.2f + (float)((2 * sp + 1) * M * N) * (4.f / 4.6e6f);
-      if (shape < 0 || us < best) {
-        best = us;
-        shape = t;
-        splits = sp;
-      }
-    }
-  }
-}
+constexpr TileModel kModel = {kTiles, kTileShapes, 0.89f, 1.f / 4.6f};
 }  // namespace
 
 // Workspace bytes of the X pieces of an M x K matrix (the piece planes, the
@@ -545,7 +504,8 @@ hipError_t launch_matmul_h(const aq_matrix *m, const float *X, int64_t M, float 
   }
   const bool prep = rows16 && getenv("AQ_MATMUL_X_PREP");
   const int kind = kq ? 0 : q6 ? 1 : 2;
-  if (!rows16) choose_tile(kind, M, N, units, cus, m_invariant ? 1 : 16, shape, splits);
+  if (!rows16)
+    choose_tile(kModel, kind, M, N, units, 4, 2, cus, m_invariant ? 1 : 16, shape, splits);
   rows16 = rows16 && !prep;
   // AQ_MATMUL_TILE (tests): the shape itself, where the kind has it
   if (const char *env = rows16 ? nullptr : getenv("AQ_MATMUL_TILE")) {

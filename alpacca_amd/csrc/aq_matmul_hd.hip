@@ -45,44 +45,11 @@
 #include <type_traits>
 
 #include "aq_internal.h"
+#include "aq_matmul_dma.h"
 #include "aq_matmul_h.h"
 
 namespace aq {
 namespace {
-
-// ---- DMA into LDS ------------------------------------------------------------
-// 16 bytes per lane from base + voff (per lane) to LDS bytes lds + 16 * lane.
-// Written in assembly because the compiler makes every later LDS read wait
-// for the whole of an LDS DMA it knows of; the kernel waits itself
-// (dma_barrier) before the barrier that publishes a stage.  There are no
-// output registers, and the address registers are read at issue.  M0 (the LDS
-// base) has no other user in this kernel.
-__device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, const void *base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(lds), "v"(voff), "s"(base)
-               : "memory");
-}
-// 4 bytes per lane
-__device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, const void *base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-               :
-               : "s"(lds), "v"(voff), "s"(base)
-               : "memory");
-}
-// all but the last LEFT of this wave's DMAs have landed, its LDS reads are
-// done, and so are those of every other wave of the workgroup
-template <int LEFT>
-__device__ __forceinline__ void dma_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LEFT) : "memory");
-}
-__device__ __forceinline__ uint32_t lds_offset(const uint8_t *p) {
-  return (uint32_t)(size_t)(const __attribute__((address_space(3))) uint8_t *)p;
-}
-template <class V>
-__device__ __forceinline__ V lds_read(const uint8_t *p) {
-  return *reinterpret_cast<const V *>(p);
-}
 
 // ---- formats -------------------------------------------------------------------
 // The packed bytes of a 256-column group of one row in LDS: three fields one
@@ -277,16 +244,9 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
   const int g = lane >> 4, c16 = lane & 15;
-  // tiles: XCD x (workgroup id modulo 8) takes a contiguous run of them, in
-  // blocks of four M tiles times all N tiles, M tiles first: the workgroups
-  // of an XCD share X rows and weights in its L2 (16384 x 2048 at M = 2048:
-  // 272 us with all M tiles of an N tile in a row, 263 in blocks of four)
-  const int tiles = m_tiles * n_tiles, per_xcd = (tiles + 7) / 8;
-  const int t = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_xcd || t >= tiles) return;
-  const int tb = t / (4 * n_tiles), rest = t - tb * 4 * n_tiles;
-  const int tm = std::min(4, m_tiles - 4 * tb);
-  const int64_t m0 = (int64_t)(4 * tb + rest % tm) * BM, n0 = (int64_t)(rest / tm) * BN;
+  int mt, nt;
+  if (!xcd_tile((int)blockIdx.x, m_tiles, n_tiles, mt, nt)) return;
+  const int64_t m0 = (int64_t)mt * BM, n0 = (int64_t)nt * BN;
   const int64_t K = (int64_t)ng * 256;
   const int b_begin = (int)blockIdx.z * per_split;
   const int b_end = std::min(b_begin + per_split, ng);

@@ -87,11 +87,13 @@ extern "C" {
 /* ---- matmul_t precision -------------------------------------------------- */
 #define AQ_PREC_AUTO 0   /* float32 accuracy (the reference's own float32
                             matmul, qmatrix.py:196-211); BF16 is opt-in      */
-#define AQ_PREC_FP32 1   /* float32 accuracy: Q4_K as exact integer weights
-                            (sc*code) on fp16 MFMA with X in two fp16 pieces
-                            (22 bits) and fp32 scales; other formats fp32
-                            MFMA over exactly decoded weights.  The same bits
-                            for any M                                        */
+#define AQ_PREC_FP32 1   /* float32 accuracy: quantized weights as exact
+                            integers on fp16 MFMA with X in two fp16 pieces
+                            (22 bits) and fp32 scales, dense weights on
+                            16-bit MFMA with the operands in exact pieces
+                            (F16: X in two, BF16 and F32: in three); the rest
+                            fp32 MFMA over exactly decoded weights.  The same
+                            bits for any M                                   */
 #define AQ_PREC_BF16 2   /* weights and X rounded to bf16, MFMA, fp32 accum.   */
 #define AQ_PREC_INT8 3   /* Q8_0 only: X quantized to int8 per 32-element block
                             (d = absmax/127, q = rint(x/d)), exact int8 MFMA
@@ -187,15 +189,15 @@ int aq_matvec_fused(const aq_matrix *const *ms, int n, const float *x,
 /* Y[M, rows] = X[M, cols] W^T.  Replaces QuantMatrix.matmul_t
  * (qmatrix.py:184-211); AQ_ERR_VALUE for M < 0.  `precision` is one of
  * AQ_PREC_*.  AQ_PREC_AUTO keeps float32 accuracy: the exact-integer fp16
- * kernels (weights as exact fp16 integers, X in two fp16 pieces) from 8
- * rows of X for Q4_K and Q5_K and from 64 rows for Q6_K, Q8_0, Q4_0, Q4_1,
- * Q5_0 and Q5_1 (K a multiple of 256 for the last five), K split over
- * workgroups where that fills the GPU; fewer rows on the integer decode
- * matvec with several rows of X sharing one weight stream (the accuracy of
- * aq_matvec; up to 32 rows, 63 for matrices of 2^24 weights or more), the
- * rest (dense matrices among them) on fp32 MFMA.  AQ_PREC_FP32 gives every
- * M the same bits (the batched prefill step's precision); AQ_PREC_BF16 is
- * an opt-in. */
+ * kernels (weights as exact fp16 integers, X in two fp16 pieces) from 3
+ * rows of X for Q4_K and Q5_K and from 5 for Q6_K, Q8_0, Q4_0, Q4_1, Q5_0
+ * and Q5_1 (K a multiple of 256 for the last five), K split over workgroups
+ * where that is faster; fewer rows on the integer decode matvec with several
+ * rows of X sharing one weight stream (the accuracy of aq_matvec; other
+ * matrices up to 32 rows, 63 for 2^24 weights or more); dense matrices of
+ * finite values on 16-bit MFMA in exact pieces (one row: the fp32 matvec);
+ * the rest on fp32 MFMA.  AQ_PREC_FP32 gives every M the same bits (the
+ * batched prefill step's precision); AQ_PREC_BF16 is an opt-in. */
 int aq_matmul_t(const aq_matrix *m, const float *X, int64_t M, float *Y,
                 int precision, int flags, void *stream);
 

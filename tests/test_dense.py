@@ -154,3 +154,60 @@ def test_model_with_dense_matrices_greedy(tmp_path, dense):
     p = tmp_path / "m.gguf"
     gguf.write_model(p, hp, tensors)
     assert gguf.load_model(p).generate_greedy(prompt, 12) == toks
+
+
+# Tile kernel (aq_matmul_dn.hip): sizes that end inside a tile of each shape and
+# inside a 64-column stage.  Bar: 2^-22 of ||W_r|| ||x_m|| from the pieces and
+# as much again for the fp32 sums.
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DENSE)
+@pytest.mark.parametrize("M,rows,cols", [(2, 1, 32), (33, 130, 96), (130, 300, 1056)])
+def test_dense_tile_shapes_vs_f64(dtype, M, rows, cols, monkeypatch):
+    data = synth.dense_values_bytes(dtype, rows, cols, seed=rows, std=1.0)
+    W = DenseMatrix(data, dtype, rows, cols)
+    ref = DenseRef(data, dtype, rows, cols)
+    X = synth.random_x(cols, seed=M, batch=M)
+    X[0] *= 1e30
+    X[1] *= 1e-30
+    want, norms = ref.matmul_t_f64(X), ref.row_norms()
+    first = None
+    for shape in range(4):
+        monkeypatch.setenv("AQ_MATMUL_TILE", str(shape))
+        for prec in ("fp32", "auto"):
+            Y = W.matmul_t(X, precision=prec)
+            err = max(normalized_error(Y[i], want[i], norms, X[i]) for i in range(M))
+            assert err < 2.0 ** -21, (shape, prec, err)
+            if prec == "fp32":
+                first = Y if first is None else first
+                assert np.array_equal(Y.view(np.uint32), first.view(np.uint32)), shape
+    assert np.array_equal(W.matmul_t(X[:1], precision="fp32").view(np.uint32),
+                          first[:1].view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DENSE)
+def test_dense_matmul_t_nonfinite(dtype):
+    """Infinities and NaNs in X and in the weights give what float32 products
+    give, and leave the other rows and columns alone."""
+    M, rows, cols = 40, 64, 128
+    w = np.random.default_rng(1).standard_normal((rows, cols)).astype(np.float32)
+    if dtype == "BF16":
+        w = (w.view(np.uint32) & 0xFFFF0000).view(np.float32)
+    X = synth.random_x(cols, seed=2, batch=M)
+    X[3, 5], X[4, 6], X[5, 7] = np.inf, -np.inf, np.nan
+    X[6, 8] = 3.4e38
+    for bad_w in (False, True):
+        if bad_w:
+            w[7, 9], w[8, 10] = np.inf, np.nan
+        data = (w.astype(np.float16).view(np.uint8) if dtype == "F16" else
+                (w.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8) if dtype == "BF16"
+                else w.view(np.uint8)).reshape(-1)
+        wv = w.astype(np.float16).astype(np.float64) if dtype == "F16" else w.astype(np.float64)
+        with np.errstate(invalid="ignore", over="ignore"):
+            want = (X.astype(np.float64) @ wv.T).astype(np.float32)
+        Y = DenseMatrix(data, dtype, rows, cols).matmul_t(X)
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isnan(want), np.isnan(Y))
+        assert np.array_equal(want[~fin & ~np.isnan(want)], Y[~fin & ~np.isnan(want)])
+        scale = np.abs(X).max(axis=1, keepdims=True) * 64
+        assert (np.abs(Y - want)[fin] < 1e-5 * np.broadcast_to(scale, Y.shape)[fin]).all()
