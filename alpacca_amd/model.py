@@ -406,12 +406,13 @@ class Model:
             self._bb = b
         return b
 
-    def _prefill_batch(self, tokens: list[int]) -> np.ndarray:
+    def _enqueue_prefill(self, tokens: list[int]) -> None:
         """The batched step over chunks of prefill_chunk tokens at positions
         n_past..: RMSNorm of all rows, matmul_t for every projection (fp32
         MFMA unless prefill_precision says otherwise), RoPE + KV store of the
         chunk, causal attention of its queries, SwiGLU, residual adds; then
-        the head on the last token only.  Returns its logits."""
+        the head on the last token only, whose logits the stream leaves in
+        self.logits."""
         hp, torch = self.hp, self.torch
         if self.n_past + len(tokens) > self.n_ctx:
             raise RuntimeError(f"context window full ({self.n_ctx} tokens)")
@@ -468,8 +469,12 @@ class Model:
                 self.n_past += T
             self.x.copy_(X[T - 1])
             self._enqueue_head()
-        self.stream.synchronize()
         self.cached_ids.extend(tokens)
+
+    def _prefill_batch(self, tokens: list[int]) -> np.ndarray:
+        """_enqueue_prefill, awaited; returns the last token's logits."""
+        self._enqueue_prefill(tokens)
+        self.stream.synchronize()
         return self.logits.cpu().numpy()
 
     def _run_prompt(self, tokens: list[int]) -> None:
@@ -500,12 +505,12 @@ class Model:
         logits = forward(token) ...).  Starts from an empty cache.  The
         prompt runs through the batched step (batch_prefill=True) or through
         the decode step; every generated token after the first is one decode
-        step.  With graph=True the steps run as HIP graph replays of
-        steps_per_graph steps each (the state advances on the device, so the
-        steps are identical; one replay of a one-step graph per token for the
-        remainder): 1807-1815 tok/s on the 1B model at 8-64 steps per graph
-        against 1791-1793 at one.  `timing`, if given,
-        receives the elapsed milliseconds of those n_gen - 1 decode steps
+        step.  With graph=True the steps run as HIP graph replays, one step
+        each, and where there are at least four times steps_per_graph of
+        them, from twice steps_per_graph on, steps_per_graph steps each (the
+        state advances on the device, so the steps are identical):
+        1807-1815 tok/s on the 1B model at 8-64 steps per graph against
+        1791-1793 at one.  `timing`, if given, receives the elapsed milliseconds of those n_gen - 1 decode steps
         (HIP events on the launch stream), their count, and the wall time of
         the prompt (prefill_ms).
 
@@ -549,15 +554,12 @@ class Model:
             advance()
 
         per_graph = max(1, int(steps_per_graph))
-        run_prompt, run_gen, run_gen_k = prompt_step, gen_step, None
-        if graph:  # captured first: the captures' eager warmup steps write junk
+        run_prompt, run_gen = prompt_step, gen_step
+        # hist and window are filled on the caller's stream
+        self.stream.wait_stream(torch.cuda.current_stream(self.dev))
+        if graph:  # captured first: the capture's eager warmup step writes junk
             g_gen = self._capture(gen_step)  # that the prompt then overwrites
             run_gen = g_gen.replay
-            if per_graph > 1 and n_gen - 1 >= per_graph:
-                def gen_k():
-                    for _ in range(per_graph):
-                        gen_step()
-                run_gen_k = self._capture(gen_k).replay
             if not batch_prefill:
                 with torch.cuda.stream(self.stream):
                     self._set_state(prompt[0], 0, fed=1)
@@ -565,34 +567,62 @@ class Model:
                 run_prompt = g_prompt.replay
         import time
         t_pf = time.perf_counter()
-        if batch_prefill:
-            self._prefill_batch(list(prompt))  # logits of the last prompt token
-        else:
+        try:
             with torch.cuda.stream(self.stream):
-                self._set_state(prompt[0], 0, fed=1)
-                for _ in range(n_p - 1):
-                    run_prompt()
-                self._enqueue_layers()  # the last prompt token, with its logits
-                self._enqueue_head()
+                if batch_prefill:
+                    # state of the first token below (the batched step reads
+                    # none), copied before the prompt's launches: the copy
+                    # waits for the stream
+                    self._set_state(0, n_p - 1, fed=0, count=0)
+                    if window is not None:
+                        window.copy_(torch.from_numpy(ring))
+                    self._enqueue_prefill(list(prompt))
+                else:
+                    self._set_state(prompt[0], 0, fed=1)
+                    for _ in range(n_p - 1):
+                        run_prompt()
+                    self._enqueue_layers()  # the last prompt token, with its logits
+                    self._enqueue_head()
+                if timing is not None:
+                    self.stream.synchronize()
+                    t_pf = time.perf_counter() - t_pf
+                # the first token: argmax of the prompt's logits; state at the
+                # last prompt position, prompt consumed
+                if not batch_prefill:
+                    self._set_state(0, n_p - 1, fed=0, count=0)
+                    if window is not None:
+                        window.copy_(torch.from_numpy(ring))
+                advance()
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record(self.stream)
+                left = n_gen - 1
+                # Graphs of per_graph steps from four graphs' worth of steps on:
+                # twice per_graph steps run as single replays, and the host
+                # captures the longer graph while they do (0.13 ms per step of
+                # four 1B-shaped layers, where a step takes 0.135 ms and its
+                # replay 0.035 ms of host time; after per_graph steps only,
+                # the device waited 0.7 ms for it).  Captured ahead of the
+                # prompt with an eager warmup run of its own it cost 4.6 ms
+                # before the first token: calls of 48 / 128 / 256 tokens
+                # after 200 took 13.6 / 24.6 / 42.7 ms and take 8.3 / 19.5 /
+                # 37.4, and 8.3 / 20.2 / 39.0 with single replays throughout.
+                if graph and 1 < per_graph <= left // 4:
+                    for _ in range(2 * per_graph):
+                        run_gen()
+                    left -= 2 * per_graph
+
+                    def gen_k():
+                        for _ in range(per_graph):
+                            gen_step()
+                    g_gen_k = self._capture_warm(gen_k)
+                    while left >= per_graph:
+                        g_gen_k.replay()
+                        left -= per_graph
+                for _ in range(left):
+                    run_gen()
+                b.record(self.stream)
+        finally:  # hist, window and the graphs are in use until here
             self.stream.synchronize()
-        t_pf = time.perf_counter() - t_pf
-        with torch.cuda.stream(self.stream):
-            # the first token: argmax of the prompt's logits; state at the
-            # last prompt position, prompt consumed
-            self._set_state(0, n_p - 1, fed=0, count=0)
-            if window is not None:
-                window.copy_(torch.from_numpy(ring))
-            advance()
-            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            a.record(self.stream)
-            left = n_gen - 1
-            while run_gen_k is not None and left >= per_graph:
-                run_gen_k()
-                left -= per_graph
-            for _ in range(left):
-                run_gen()
-            b.record(self.stream)
-        self.stream.synchronize()
         if timing is not None:
             timing["gen_ms"] = a.elapsed_time(b)
             timing["steps"] = n_gen - 1
@@ -613,6 +643,21 @@ class Model:
         with torch.cuda.graph(g, stream=self.stream):
             fn()
         self.stream.synchronize()
+        return g
+
+    def _capture_warm(self, fn):
+        """A HIP graph of fn on self.stream, for launches that the stream has
+        run before (their workspace is there).  Work queued on the stream
+        runs on meanwhile: unlike torch.cuda.graph, nothing here waits for
+        the device."""
+        torch = self.torch
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(self.stream):
+            g.capture_begin()
+            try:
+                fn()
+            finally:
+                g.capture_end()
         return g
 
 

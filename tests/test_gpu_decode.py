@@ -440,9 +440,9 @@ def test_tiny_model_greedy_tokens(tiny, graph, batch_prefill):
 @pytest.mark.parametrize("per_graph", [1, 5, 39, 40])
 def test_tiny_model_greedy_steps_per_graph(tiny, per_graph):
     """Replays of a graph of several decode steps give the tokens of one step
-    per replay: 39 steps after the first token run as 7 x 5 + 4, 1 x 39, and
-    39 single replays where the multi-step graph would be longer than the
-    run (40)."""
+    per replay: 39 steps after the first token run as 10 + 5 x 5 + 4, and as
+    single replays where four of the longer graphs would exceed the run
+    (39, 40)."""
     print(f"tiny model greedy steps_per_graph={per_graph}", flush=True)
     hp, tensors = tiny
     prompt = list(np.random.default_rng(2).integers(0, hp.n_vocab, 60))
@@ -455,6 +455,24 @@ def test_tiny_model_greedy_steps_per_graph(tiny, per_graph):
     # and the model continues from there like after single-step replays
     got2 = gm.generate_greedy(prompt[:30], 12, steps_per_graph=per_graph)
     assert got2 == MR.RefModel(hp, tensors).greedy(prompt[:30], 12)[0]
+
+
+@pytest.mark.parametrize("n_gen", [16, 20, 21, 23, 26])
+def test_tiny_model_greedy_multi_step_graph(tiny, n_gen):
+    """The multi-step graph is captured while single-step replays run, from
+    four graphs' worth of steps on (5 steps each: 15 and 19 steps run singly,
+    20 as 10 + 2 x 5, 22 with 2 left over, 25 as 10 + 3 x 5), with and
+    without the penalty window, and after a longer prompt's call has grown
+    the stream's workspace."""
+    print(f"tiny model greedy multi-step graph n_gen={n_gen}", flush=True)
+    hp, tensors = tiny
+    rng = np.random.default_rng(n_gen)
+    gm, ref = Model(hp, tensors), MR.RefModel(hp, tensors)
+    for t, kw in ((9, {}), (90, dict(repeat_penalty=1.1, repeat_last_n=8)), (30, {})):
+        prompt = list(rng.integers(0, hp.n_vocab, t))
+        assert gm.generate_greedy(prompt, n_gen, steps_per_graph=5, **kw) == \
+            ref.greedy(prompt, n_gen, **kw)[0], (t, kw)
+        assert gm.n_past == t + n_gen - 1
 
 
 @pytest.mark.parametrize("graph", [True, False])
