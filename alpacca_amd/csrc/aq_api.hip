@@ -835,8 +835,9 @@ int matmul_t_impl(const aq_matrix *m, const float *X, int64_t M, float *Y, int p
                                                     (precision == AQ_PREC_AUTO && M >= exact_min));
   // Dense weights: 16-bit matrix cores at float32 accuracy (aq_matmul_dn.hip;
   // FP32 again without a split of K), one row at AUTO the fp32 matvec (14336
-  // x 4096: F16 22 us against 27, F32 42 against 45).
-  const bool dense1 = precision == AQ_PREC_AUTO && M == 1 && aq::is_dense(m->dtype);
+  // x 4096: F16 22 us against 27, F32 42 against 45) where it holds x in LDS.
+  const bool dense1 = precision == AQ_PREC_AUTO && M == 1 && aq::is_dense(m->dtype) &&
+                      aq::matvec_one_launch(m);
   const bool dense16 = !dense1 && (precision == AQ_PREC_AUTO || precision == AQ_PREC_FP32) &&
                        aq::mm_dn_supported(m);
   const bool small = !exact_fp16 && precision == AQ_PREC_AUTO && M <= (big ? 63 : 32) &&

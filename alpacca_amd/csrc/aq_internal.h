@@ -104,6 +104,8 @@ void release_workspace(hipStream_t s);
 
 // Largest K (columns) the matvec kernel accepts: x is staged whole in LDS.
 int64_t matvec_max_cols(int dtype, int device);
+// whether this matrix's rows are no wider
+bool matvec_one_launch(const aq_matrix *m);
 
 // Integer-dot decode matvec (aq_matvec_i8.hip): LDS bytes of the prepared x
 // of one row, the largest K it accepts, and the launcher (x -> y).

@@ -252,37 +252,38 @@ hipError_t launch_fmt(const aq_matrix *m, const float *x, float *y,
 
 }  // namespace
 
+// bytes of LDS of a row of nb blocks: x (4 per column), half-chunk sums (8
+// per chunk), padding of the last 64-chunk group; 0 for an unknown format
+static size_t lds_bytes_of(int dtype, int64_t nb) {
+  switch (dtype) {
+    case AQ_Q4_K: return matvec_lds_bytes<Q4K>(nb);
+    case AQ_Q5_K: return matvec_lds_bytes<Q5K>(nb);
+    case AQ_Q6_K: return matvec_lds_bytes<Q6K>(nb);
+    case AQ_Q8_0: return matvec_lds_bytes<Q80>(nb);
+    case AQ_Q4_0: return matvec_lds_bytes<Q40>(nb);
+    case AQ_Q4_1: return matvec_lds_bytes<Q41>(nb);
+    case AQ_Q5_0: return matvec_lds_bytes<Q50>(nb);
+    case AQ_Q5_1: return matvec_lds_bytes<Q51>(nb);
+    case AQ_F32: return matvec_lds_bytes<F32D>(nb);
+    case AQ_F16: return matvec_lds_bytes<F16D>(nb);
+    case AQ_BF16: return matvec_lds_bytes<BF16D>(nb);
+    default: return 0;
+  }
+}
+
+bool matvec_one_launch(const aq_matrix *m) {
+  const size_t need = lds_bytes_of(m->dtype, m->nb_row);
+  return need > 0 && need <= device_info(m->device).lds_max;
+}
+
 int64_t matvec_max_cols(int dtype, int device) {
   const size_t lds = device_info(device).lds_max;
-  // bytes of LDS per column: x (4) + half-chunk sums (8 per chunk) + padding
-  // of the last 64-chunk group; solve conservatively per format.
-  int64_t be = 256;
-  switch (dtype) {
-    case AQ_Q4_0: case AQ_Q4_1: case AQ_Q5_0: case AQ_Q5_1: case AQ_Q8_0:
-    case AQ_F32: case AQ_F16: case AQ_BF16:
-      be = 32;
-      break;
-    default:
-      break;
-  }
+  const bool k256 = dtype == AQ_Q4_K || dtype == AQ_Q5_K || dtype == AQ_Q6_K;
+  const int64_t be = k256 ? 256 : 32;
   int64_t k = 0;
   for (int64_t cand = be; cand <= (int64_t)1 << 20; cand += be) {
-    size_t need = 0;
-    const int64_t nb = cand / be;
-    switch (dtype) {
-      case AQ_Q4_K: need = matvec_lds_bytes<Q4K>(nb); break;
-      case AQ_Q5_K: need = matvec_lds_bytes<Q5K>(nb); break;
-      case AQ_Q6_K: need = matvec_lds_bytes<Q6K>(nb); break;
-      case AQ_Q8_0: need = matvec_lds_bytes<Q80>(nb); break;
-      case AQ_Q4_0: need = matvec_lds_bytes<Q40>(nb); break;
-      case AQ_Q4_1: need = matvec_lds_bytes<Q41>(nb); break;
-      case AQ_Q5_0: need = matvec_lds_bytes<Q50>(nb); break;
-      case AQ_Q5_1: need = matvec_lds_bytes<Q51>(nb); break;
-      case AQ_F32: need = matvec_lds_bytes<F32D>(nb); break;
-      case AQ_F16: need = matvec_lds_bytes<F16D>(nb); break;
-      case AQ_BF16: need = matvec_lds_bytes<BF16D>(nb); break;
-      default: return 0;
-    }
+    const size_t need = lds_bytes_of(dtype, cand / be);
+    if (need == 0) return 0;
     if (need > lds) break;
     k = cand;
   }

@@ -211,3 +211,16 @@ def test_dense_matmul_t_nonfinite(dtype):
         assert np.array_equal(want[~fin & ~np.isnan(want)], Y[~fin & ~np.isnan(want)])
         scale = np.abs(X).max(axis=1, keepdims=True) * 64
         assert (np.abs(Y - want)[fin] < 1e-5 * np.broadcast_to(scale, Y.shape)[fin]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DENSE)
+def test_dense_matmul_t_one_wide_row(dtype):
+    """One row of X wider than the matvec kernel stages in LDS (K = 53,248 is a
+    405B-class ffn_down) runs as well."""
+    rows, cols = 3, 53248
+    data = synth.dense_values_bytes(dtype, rows, cols, seed=1, std=1.0)
+    W, ref = DenseMatrix(data, dtype, rows, cols), DenseRef(data, dtype, rows, cols)
+    X = synth.random_x(cols, seed=2, batch=1)
+    err = normalized_error(W.matmul_t(X)[0], ref.matmul_t_f64(X)[0], ref.row_norms(), X[0])
+    assert err < 2.0 ** -21, err
