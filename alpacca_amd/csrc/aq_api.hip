@@ -411,6 +411,11 @@ void *workspace(int device, hipStream_t s, size_t bytes) {
   return p;
 }
 
+void workspace_forgo() {
+  g_ws_refused_capture = false;
+  (void)hipGetLastError();
+}
+
 void release_workspace(hipStream_t s) {
   std::lock_guard<std::mutex> lock(g_ws_mu);
   for (size_t i = 0; i < g_ws_live.size();) {
@@ -881,9 +886,16 @@ int matmul_t_impl(const aq_matrix *m, const float *X, int64_t M, float *Y, int p
           e = aq::launch_matvec(m, static_cast<const float *>(din), yo, s);
         } else if (dense16) {  // in slices of rows for the same reason
           const int64_t rows_max = std::max<int64_t>(1, ((int64_t)1 << 29) / (m->cols + 32));
-          for (int64_t r0 = 0; r0 < M && e == hipSuccess; r0 += rows_max)
-            e = aq::launch_matmul_dn(m, static_cast<const float *>(din) + r0 * m->cols,
-                                     std::min(rows_max, M - r0), yo + r0 * m->rows, m_invariant, s);
+          for (int64_t r0 = 0; r0 < M && e == hipSuccess; r0 += rows_max) {
+            const float *x = static_cast<const float *>(din) + r0 * m->cols;
+            const int64_t mr = std::min(rows_max, M - r0);
+            bool no_scratch = false;
+            e = aq::launch_matmul_dn(m, x, mr, yo + r0 * m->rows, m_invariant, s, &no_scratch);
+            if (no_scratch) {  // the fp32 matrix cores, which need none from about 4,096 weight rows on
+              aq::workspace_forgo();
+              e = aq::launch_matmul_t(m, x, mr, yo + r0 * m->rows, precision, s);
+            }
+          }
         } else if (small) {
           e = aq::launch_matvec_i8_batch(m, static_cast<const float *>(din), M, m->cols, yo,
                                          m->rows, s);

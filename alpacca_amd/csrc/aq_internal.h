@@ -82,11 +82,15 @@ hipError_t launch_matmul_h(const aq_matrix *m, const float *X, int64_t M, float 
 // matmul_t of dense weights on 16-bit matrix cores at float32 accuracy
 // (aq_matmul_dn.hip), for matrices without infinities and NaNs
 // (mm_dn_supported; dense_all_finite looks through a matrix's device copy).
-// m_invariant as for launch_matmul_h.
+// m_invariant as for launch_matmul_h.  *no_scratch: nothing was launched, since
+// the stream's workspace cannot hold the pieces of X.
 bool mm_dn_supported(const aq_matrix *m);
 hipError_t dense_all_finite(const aq_matrix *m, bool *finite);
 hipError_t launch_matmul_dn(const aq_matrix *m, const float *X, int64_t M, float *Y,
-                            bool m_invariant, hipStream_t s);
+                            bool m_invariant, hipStream_t s, bool *no_scratch);
+// Takes back the notes of a refused workspace (a capture's, HIP's last
+// error), for a caller that goes on without one.
+void workspace_forgo();
 
 // Device scratch memory for work on stream `s` of `device`, at least `bytes`
 // long (nullptr when it cannot be allocated).  One buffer per (device,

@@ -415,7 +415,8 @@ bool mm_dn_supported(const aq_matrix *m) {
 }
 
 hipError_t launch_matmul_dn(const aq_matrix *m, const float *X, int64_t M, float *Y,
-                            bool m_invariant, hipStream_t s) {
+                            bool m_invariant, hipStream_t s, bool *no_scratch) {
+  *no_scratch = false;
   if (M == 0 || m->rows == 0) return hipSuccess;
   const int kind = m->dtype == AQ_F16 ? kF16 : m->dtype == AQ_BF16 ? kBF16 : kF32;
   const int64_t K = m->cols, N = m->rows, Kp = (K + 63) / 64 * 64;
@@ -435,7 +436,10 @@ hipError_t launch_matmul_dn(const aq_matrix *m, const float *X, int64_t M, float
   const size_t xb = al((size_t)pieces_of(kind) * plane * 2), eb = al((size_t)M * 4);
   const size_t part = splits > 1 ? (size_t)splits * M * N * 4 : 0;
   uint8_t *ws = static_cast<uint8_t *>(workspace(m->device, s, xb + eb + part));
-  if (!ws) return hipErrorOutOfMemory;
+  if (!ws) {
+    *no_scratch = true;
+    return hipErrorOutOfMemory;
+  }
   uint16_t *xp = reinterpret_cast<uint16_t *>(ws);
   int32_t *xe = reinterpret_cast<int32_t *>(ws + xb);
   float *dst = splits > 1 ? reinterpret_cast<float *>(ws + xb + eb) : Y;

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from alpacca_amd import _lib, synth
-from alpacca_amd.qmatrix import QuantMatrix
+from alpacca_amd.qmatrix import DenseMatrix, QuantMatrix
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -82,3 +82,32 @@ def test_capture_refuses_scratch_growth():
     s.synchronize()
     ref = qm.matmul_t(X.cpu().numpy())
     assert np.array_equal(Y.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dtype", ["F16", "BF16", "F32"])
+def test_dense_capture_without_scratch(dtype):
+    """A dense matmul_t captured on a stream that holds no scratch runs on the
+    fp32 matrix cores, which need none for this many weight rows; the error
+    of a call that does need some is not left behind.  Bar 1e-5 of max|Y|
+    between the two kernels' fp32 sums over 256 columns."""
+    d = torch.device("cuda", 0)
+    rows, cols, M = 4224, 256, 5
+    W = DenseMatrix(synth.dense_values_bytes(dtype, rows, cols, seed=4), dtype, rows, cols)
+    X = torch.from_numpy(synth.random_x(cols, seed=5, batch=M)).to(d)
+    want = W.matmul_t(X.cpu().numpy())
+    Y = torch.empty((M, rows), device=d)
+    s = torch.cuda.Stream(d)
+    h = s.cuda_stream
+    _lib.check(_lib.ensure_device().aq_release_workspace(ctypes.c_void_p(h)))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        W.matmul_t_device(X.data_ptr(), M, Y.data_ptr(), h)
+    for _ in range(3):
+        Y.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            g.replay()
+        s.synchronize()
+        assert np.abs(Y.cpu().numpy() - want).max() < 1e-5 * np.abs(want).max()
+    with pytest.raises(ValueError):  # its own message, not the refused scratch
+        W.matmul_t_device(X.data_ptr(), -1, Y.data_ptr(), h)
