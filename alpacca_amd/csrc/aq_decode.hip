@@ -873,8 +873,8 @@ __global__ void __launch_bounds__(256)
 // accumulator (what is dropped is below 2^-25 of it), so products and sums
 // keep fp32's accuracy at 6/16 of the fp32 matrix cores' time
 // (v_mfma_f32_16x16x32_bf16 against 16x16x4f32).  No scaling is needed: bf16
-// has fp32's exponent range.  A non-finite q, K or V makes the rows that see it
-// non-finite.
+// has fp32's exponent range.  Rows that meet an infinity or a NaN are formed
+// again in fp32 at the end.
 //
 // Grid: one workgroup of NW waves per (16 NW (token, head) rows, kv head); a
 // wave owns 16 rows (16 / G tokens times the G heads) and keeps the online
@@ -889,8 +889,8 @@ __global__ void __launch_bounds__(256)
 //     4 g .. +3 and 32 u + 16 + 4 g .. +3; V^T's columns are stored in that
 //     order).  The weights' pieces are cut by truncation (exact).
 //
-// 32 / 8 heads of 64, 2048 tokens (a 1B layer): 257 us on fp32 matrix cores,
-// 119 here; of 128, 609 -> 205; 100 tokens at position 1000 62 -> 44 and 128 ->
+// 32 / 8 heads of 64, 2048 tokens (a 1B layer): 253 us on fp32 matrix cores,
+// 102 here; of 128, 609 -> 205; 100 tokens at position 1000 62 -> 44 and 128 ->
 // 76; error against float64 4.0e-7 -> 2.9e-7 and 4.5e-7 -> 3.0e-7.  What bounds
 // it: per wave and chunk of 64 dimensions 96 matrix products (1,536 cycles)
 // and about as many cycles of VALU (softmax and the pieces of the weights, 800;
@@ -1111,6 +1111,51 @@ __global__ void __launch_bounds__(64 * NW)
   // lane (r16, cg) of tile ht holds O^T[16 ht + 4 cg + r][row r16]
   float den = add_xor<16>(l);
   den = add_xor<32>(den);
+  // Rows whose pieces were not finite (an infinity leaves inf - inf, a value
+  // within 2^-9 of the largest rounds up to one, and what is masked for the row
+  // counts too) come out NaN and are formed again in fp32 over what they see.
+  float chk = den - den;
+#pragma unroll
+  for (int ht = 0; ht < NHT; ++ht)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) chk = fmaf(o[ht][r], 0.f, chk);
+  const bool again = t_row < T && add_xor<32>(add_xor<16>(chk)) != 0.f;
+  if (__any(again)) {
+#pragma clang fp contract(off)  // (d - mn of the maximum itself is 0, not d's rounding)
+    int64_t last = -1;          // the row's last position
+    if (again) last = pb + t_row < n_ctx ? pb + t_row : n_ctx - 1;
+    const f4v_ *qr = reinterpret_cast<const f4v_ *>(
+        q + ((t_row < T ? t_row : T - 1) * n_head + h_row) * HD);
+    f4v_ a[NHT];
+#pragma unroll
+    for (int ht = 0; ht < NHT; ++ht) a[ht] = f4v_{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, ls = 0.f;
+#pragma unroll 1
+    for (int64_t pg = 0; pg <= p_last; ++pg) {  // the same for all lanes of the wave
+      float d = 0.f;
+#pragma unroll
+      for (int ht = 0; ht < NHT; ++ht) {
+        const f4v_ qv = qr[4 * ht + cg], kv = kb[pg * D4 + 4 * ht + cg];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d = fmaf(qv[r], kv[r], d);
+      }
+      d = add_xor<32>(add_xor<16>(d)) * scale;
+      if (pg > last) continue;
+      const float mn = fmaxf(m, d), c0 = mn == -INFINITY ? 0.f : mn;
+      const float corr = m == -INFINITY ? 0.f : expf(m - mn), e = expf(d - c0);
+      ls = fmaf(ls, corr, e);
+#pragma unroll
+      for (int ht = 0; ht < NHT; ++ht)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a[ht][r] = fmaf(e, vb[pg * D4 + 4 * ht + cg][r], a[ht][r] * corr);
+      m = mn;
+    }
+    if (again) {
+      den = ls;
+#pragma unroll
+      for (int ht = 0; ht < NHT; ++ht) o[ht] = a[ht];
+    }
+  }
   if (t_row < T) {
     const float inv = 1.f / den;
 #pragma unroll

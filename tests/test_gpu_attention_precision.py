@@ -97,3 +97,46 @@ def test_attention_batch_three_pieces_vs_f64(hd, T, vscale, qscale):
         want = (w / w.sum(axis=1, keepdims=True)) @ V[kv].astype(np.float64)
         err = np.abs(whole[:, h * hd:(h + 1) * hd] - want).max() / np.abs(V).max()
         assert err < 1e-5, (h, err)
+
+
+@pytest.mark.parametrize("hd,T", [(64, 100), (128, 70), (64, 2)])
+def test_attention_batch_nonfinite(hd, T):
+    """Infinities and NaNs in q, K and V, and finite values that round to a
+    bf16 infinity, give what the float32 softmax over the positions a row sees
+    gives (a score of -inf is a weight of zero), and leave the rows that do not
+    see them alone.  Bar 1e-5 max|V| of each dimension, as above."""
+    n_head, n_kv, pos0 = 8, 2, 9
+    n_ctx = pos0 + T
+    rng = np.random.default_rng(hd * T)
+    q = rng.standard_normal((T, n_head, hd)).astype(np.float32)
+    K = rng.standard_normal((n_kv, n_ctx, hd)).astype(np.float32)
+    V = rng.standard_normal((n_kv, n_ctx, hd)).astype(np.float32)
+    q[..., 0], q[..., 1] = 1.0, np.float32(2.0 ** -126)
+    K[0, 2, 0] = -np.inf                      # no weight
+    K[0, 4, 1] = np.finfo(np.float32).max     # adds 4 to the score
+    V[0, 5, 3] = np.inf                       # that dimension infinite
+    V[1, 6, 7] = np.finfo(np.float32).max     # finite products
+    if T > 60:
+        V[1, pos0 + 40, 2] = np.nan           # seen from token 40 on
+        q[50, 3, 5] = np.nan
+        q[20, 1, 2] = np.inf
+    qd, kc, vc = (torch.from_numpy(a).to("cuda") for a in (q, K, V))
+    out = torch.empty((T, n_head, hd), device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    _lib.check(_lib.ensure_device().aq_attention_batch(p(qd), p(kc), p(vc), T, n_head, n_kv, hd,
+                                                       n_ctx, None, pos0, p(out), None))
+    got = out.cpu().numpy()
+    with np.errstate(all="ignore"):
+        for t in range(T):
+            n = pos0 + t + 1
+            for h in range(n_head):
+                kv = h // (n_head // n_kv)
+                s = (K[kv, :n].astype(np.float64) @ q[t, h].astype(np.float64)) / math.sqrt(hd)
+                w = np.exp(s - s.max())
+                want = (w / w.sum()) @ V[kv, :n].astype(np.float64)
+                fin = np.isfinite(want)
+                g = got[t, h]
+                assert np.array_equal(np.isnan(want), np.isnan(g)), (t, h)
+                assert np.array_equal(want[~fin], g[~fin], equal_nan=True), (t, h)
+                bar = np.abs(V[kv, :n].astype(np.float64)).max(axis=0)
+                assert (np.abs(g - want)[fin] <= 1e-5 * bar[fin]).all(), (t, h)
