@@ -496,7 +496,7 @@ def decode_leg(hp=None, tensors=None) -> dict:
     (alpacca_amd.model.synthetic_llama_1b, seed 0): a 2048-token seeded
     prompt fills the fp32 KV cache, then 256 greedy tokens; each token is
     one HIP-graph replay of the device-resident step.  The prompt runs
-    through the batched step (fp32 MFMA matmuls, one 2048-token chunk;
+    through the batched step (float32 accuracy, one 2048-token chunk;
     bit-identical to the reference's 256-token chunks); the first token is
     the argmax of its logits, and each of the other 255 is one graph
     replay.  tokens/s = 255 /
