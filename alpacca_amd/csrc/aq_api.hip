@@ -352,6 +352,11 @@ struct WsEntry {
   bool captured;  // handed out while the stream was capturing a graph
 };
 std::mutex g_ws_mu;
+std::mutex g_ws_stream_mu[64];  // WorkspaceGuard: by device and stream
+std::mutex &ws_stream_mutex(int device, hipStream_t s) {
+  const uint64_t h = ((uint64_t)(uintptr_t)s + (uint64_t)device * 977) * 0x9E3779B97F4A7C15ull;
+  return g_ws_stream_mu[h >> 58];
+}
 std::vector<WsEntry> g_ws_live;     // one buffer per (device, stream)
 std::vector<void *> g_ws_retired;   // buffers a captured graph may still use
 
@@ -374,6 +379,11 @@ void ws_drop(WsEntry &e, bool capturing_now) {
   e.captured = false;
 }
 }  // namespace
+
+WorkspaceGuard::WorkspaceGuard(int device, hipStream_t s) : mu_(ws_stream_mutex(device, s)) {
+  mu_.lock();
+}
+WorkspaceGuard::~WorkspaceGuard() { mu_.unlock(); }
 
 void *workspace(int device, hipStream_t s, size_t bytes) {
   // sizes grow geometrically (powers of two from 1 MiB), so a run of
@@ -417,17 +427,18 @@ void workspace_forgo() {
 }
 
 void release_workspace(hipStream_t s) {
-  std::lock_guard<std::mutex> lock(g_ws_mu);
-  for (size_t i = 0; i < g_ws_live.size();) {
-    if (g_ws_live[i].stream == s) {
+  for (int device = 0; device < kMaxDev; ++device) {
+    WorkspaceGuard guard(device, s);
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    for (size_t i = 0; i < g_ws_live.size(); ++i) {
+      if (g_ws_live[i].device != device || g_ws_live[i].stream != s) continue;
       int prev = 0;
       (void)hipGetDevice(&prev);
-      (void)hipSetDevice(g_ws_live[i].device);
+      (void)hipSetDevice(device);
       ws_drop(g_ws_live[i], false);
       (void)hipSetDevice(prev);
       g_ws_live.erase(g_ws_live.begin() + i);
-    } else {
-      ++i;
+      break;  // one buffer per (device, stream)
     }
   }
 }
@@ -860,6 +871,7 @@ int matmul_t_impl(const aq_matrix *m, const float *X, int64_t M, float *Y, int p
   return run_staged(
       m, X, (size_t)M * m->cols * 4, Y, (size_t)M * m->rows * 4, flags, stream,
       [&](const void *din, void *dout, hipStream_t s) {
+        aq::WorkspaceGuard guard(m->device, s);
         float *yo = static_cast<float *>(dout);
         // the SwiGLU pairs of rows r0 .. r0 + mr of Y
         auto pairs = [&](int64_t r0, int64_t mr) {
@@ -1029,6 +1041,7 @@ int aq_attention_batch(const float *q, const float *k_cache, const float *v_cach
     return e == hipSuccess ? AQ_OK : hip_fail(e, "attention launch");
   }
   const size_t bytes = aq::attention_scratch_bytes(n_kv, head_dim, n_head / n_kv, n_ctx, T);
+  aq::WorkspaceGuard guard(dev, s);
   float *part = static_cast<float *>(aq::workspace(dev, s, bytes));
   if (!part) return fail(AQ_ERR_RUNTIME, "out of device memory for attention partials");
   hipError_t e = aq::launch_attention(q, k_cache, v_cache, n_head, n_kv, head_dim, n_ctx,
@@ -1138,6 +1151,7 @@ int aq_attention_rope(float *q, const float *k, const float *v, int n_head,
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const size_t bytes = aq::attention_scratch_bytes(n_kv, head_dim, n_head / n_kv, n_ctx, 1);
+  aq::WorkspaceGuard guard(dev, s);
   float *part = static_cast<float *>(aq::workspace(dev, s, bytes));
   if (!part) return fail(AQ_ERR_RUNTIME, "out of device memory for attention partials");
   hipError_t e = aq::launch_attention_rope(q, k, v, n_head, n_kv, head_dim, n_rot,

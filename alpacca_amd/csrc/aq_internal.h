@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "../../include/alpacca_amd.h"
 #include "aq_formats.h"
 
@@ -100,11 +102,28 @@ void workspace_forgo();
 // nullptr (and the C ABI reports that the call must first run eagerly).  An
 // outgrown buffer is freed after the stream's queued work, unless it was
 // handed out during a capture: such a buffer is kept until the process
-// exits, so the graph stays valid.
+// exits, so the graph stays valid.  The buffer is the caller's only while it
+// holds the stream's WorkspaceGuard.
 void *workspace(int device, hipStream_t s, size_t bytes);
 // Drop the workspace of stream `s` (all devices), as workspace() drops an
 // outgrown buffer; the next call on the stream allocates anew.
 void release_workspace(hipStream_t s);
+// Held from workspace() until the last launch that uses the buffer is on the
+// stream: host threads that call on one stream (every call on host arrays runs
+// on the null stream) otherwise interleave their launches over the same
+// scratch, or free it by outgrowing it before another's launches are queued.
+// One at a time per thread; streams that share a lock only wait for each
+// other's enqueueing.
+class WorkspaceGuard {
+ public:
+  WorkspaceGuard(int device, hipStream_t s);
+  ~WorkspaceGuard();
+  WorkspaceGuard(const WorkspaceGuard &) = delete;
+  WorkspaceGuard &operator=(const WorkspaceGuard &) = delete;
+
+ private:
+  std::mutex &mu_;
+};
 
 // Largest K (columns) the matvec kernel accepts: x is staged whole in LDS.
 int64_t matvec_max_cols(int dtype, int device);

@@ -21,7 +21,8 @@
  * Threading: a matrix is immutable after aq_matrix_create.  Calls on
  * different streams may run concurrently; each host thread owns its own
  * staging buffers, so concurrent calls must come from different host threads
- * (or pass device pointers, which use no staging).
+ * (or pass device pointers, which use no staging).  Several threads may call on
+ * one stream too: each call's launches are queued as one, in some order.
  */
 #ifndef ALPACCA_AMD_H
 #define ALPACCA_AMD_H

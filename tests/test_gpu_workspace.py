@@ -7,6 +7,7 @@ scratch than the stream holds is refused while the stream is capturing
 from __future__ import annotations
 
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -111,3 +112,42 @@ def test_dense_capture_without_scratch(dtype):
         assert np.abs(Y.cpu().numpy() - want).max() < 1e-5 * np.abs(want).max()
     with pytest.raises(ValueError):  # its own message, not the refused scratch
         W.matmul_t_device(X.data_ptr(), -1, Y.data_ptr(), h)
+
+
+@pytest.mark.parametrize("dtype", ["F16", "F32", "Q4_K"])
+def test_threads_share_a_stream(dtype):
+    """Host threads that call on one stream (calls on host arrays all run on
+    the null stream) share its scratch: each call's pieces of X and partials
+    stay its own until its launches are queued, also while another thread's
+    larger call outgrows the buffer.  Every result has the bits of the same
+    call made alone."""
+    rows, cols = 640, 2048
+    cls = QuantMatrix if dtype == "Q4_K" else DenseMatrix
+    data = (synth.random_matrix_bytes(dtype, rows, cols, seed=6) if dtype == "Q4_K" else
+            synth.dense_values_bytes(dtype, rows, cols, seed=6))
+    W = cls(data, dtype, rows, cols)
+    # growing batches, of different sizes from thread to thread
+    Xs = [[synth.random_x(cols, seed=100 * t + i, batch=17 + 40 * i + 11 * t) for i in range(6)]
+          for t in range(4)]
+    want = [[W.matmul_t(X) for X in row] for row in Xs]
+    _lib.check(_lib.ensure_device().aq_release_workspace(None))
+    start = threading.Barrier(len(Xs))
+    bad = []
+
+    def work(t):
+        try:
+            start.wait(30)
+            for _ in range(5):
+                for X, w in zip(Xs[t], want[t]):
+                    if not np.array_equal(W.matmul_t(X).view(np.uint32), w.view(np.uint32)):
+                        bad.append((t, X.shape[0]))
+        except Exception as e:  # noqa: BLE001 (a thread's error is the test's)
+            bad.append((t, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(len(Xs))]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join(60)
+    assert not bad, bad[:8]
+    assert not any(th.is_alive() for th in threads)
