@@ -189,6 +189,8 @@ class Model:
         # aq_decode_state: int64 token, uint64 key, int32 pos, fed, count, pad
         self.state = torch.zeros(_lib.DECODE_STATE_BYTES // 4, dtype=torch.int32,
                                  device=self.dev)
+        # filled on the caller's stream, used on self.stream from here on
+        self.stream.wait_stream(torch.cuda.current_stream(self.dev))
         self.n_past = 0
         self.cached_ids: list[int] = []
         # batched prefill: chunk size (ALPACCA_PREFILL_CHUNK, model.py:630-634)
@@ -388,21 +390,24 @@ class Model:
     # ---- batched prefill (Model.forward_batch, model.py:469-518) ------------
 
     def _batch_buffers(self, T: int) -> dict:
+        """Buffers of the batched step for T tokens, on self.stream (their
+        memory is never touched by another stream's work)."""
         b = getattr(self, "_bb", None)
         if b is None or b["T"] < T:
             torch, hp = self.torch, self.hp
-            f32 = dict(dtype=torch.float32, device=self.dev)
             q_dim, kv_dim = hp.n_head * hp.head_dim, hp.n_kv * hp.head_dim
-            # GU: T x 2 n_ff, the interleaved gate/up products, or G and U
-            # (T x n_ff each) as its two halves for separate matrices
-            gu = torch.zeros(2 * T * hp.n_ff, **f32)
-            b = {"T": T, "ids": torch.zeros(T, dtype=torch.int64, device=self.dev),
-                 "X": torch.zeros((T, hp.n_embd), **f32), "H": torch.zeros((T, hp.n_embd), **f32),
-                 "O": torch.zeros((T, hp.n_embd), **f32), "Q": torch.zeros((T, q_dim), **f32),
-                 "K": torch.zeros((T, kv_dim), **f32), "V": torch.zeros((T, kv_dim), **f32),
-                 "A": torch.zeros((T, q_dim), **f32), "GU": gu.view(T, 2 * hp.n_ff),
-                 "G": gu[:T * hp.n_ff].view(T, hp.n_ff), "U": gu[T * hp.n_ff:].view(T, hp.n_ff),
-                 "S": torch.zeros((T, hp.n_ff), **f32)}
+
+            def rows(n):
+                return torch.empty((T, n), dtype=torch.float32, device=self.dev)
+            with torch.cuda.stream(self.stream):
+                # GU: T x 2 n_ff, the interleaved gate/up products, or G and U
+                # (T x n_ff each) as its two halves for separate matrices
+                gu = rows(2 * hp.n_ff).view(-1)
+                b = {"T": T, "ids": torch.empty(T, dtype=torch.int64, device=self.dev),
+                     "X": rows(hp.n_embd), "H": rows(hp.n_embd), "O": rows(hp.n_embd),
+                     "Q": rows(q_dim), "K": rows(kv_dim), "V": rows(kv_dim), "A": rows(q_dim),
+                     "GU": gu.view(T, 2 * hp.n_ff), "G": gu[:T * hp.n_ff].view(T, hp.n_ff),
+                     "U": gu[T * hp.n_ff:].view(T, hp.n_ff), "S": rows(hp.n_ff)}
             self._bb = b
         return b
 
@@ -486,8 +491,8 @@ class Model:
         if min(tokens) < 0 or max(tokens) >= self.hp.n_vocab:
             raise IndexError("row index out of range")
         torch = self.torch
-        prompt = torch.tensor(tokens, dtype=torch.int64, device=self.dev)
         with torch.cuda.stream(self.stream):
+            prompt = torch.tensor(tokens, dtype=torch.int64, device=self.dev)
             self._set_state(tokens[0], self.n_past, fed=1)
             for _ in tokens:
                 self._enqueue_layers()

@@ -510,6 +510,34 @@ def test_prefill_chunk_size_does_not_change_results(tiny):
         assert np.array_equal(lg, out[0][0]) and np.array_equal(kv, out[0][1])
 
 
+def test_prefill_behind_a_busy_caller_stream(tiny, monkeypatch):
+    """The model's buffers are made while the caller's stream is busy: what is
+    filled there is done before the model's own stream runs, and what the
+    batched step allocates for itself is not filled on the caller's stream
+    at all, so nothing lands in the middle of a prompt (300 chunks of one token
+    here, behind a sleep on the caller's stream before every fill)."""
+    hp, tensors = tiny
+    toks = list(np.random.default_rng(14).integers(0, hp.n_vocab, 300))
+    ref = Model(hp, tensors)
+    ref.prefill_chunk = 1
+    want = ref.prefill(toks), ref.forward(5), ref.kv[:, :, :, :301].cpu().numpy()
+    zeros = torch.zeros
+
+    def late_zeros(*a, **kw):
+        if "device" in kw:
+            torch.cuda._sleep(40_000_000)
+        return zeros(*a, **kw)
+    monkeypatch.setattr(torch, "zeros", late_zeros)
+    caller = torch.cuda.Stream()
+    with torch.cuda.stream(caller):
+        gm = Model(hp, tensors)
+        gm.prefill_chunk = 1
+        got = gm.prefill(toks), gm.forward(5)
+    caller.synchronize()
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    assert np.array_equal(gm.kv[:, :, :, :301].cpu().numpy(), want[2])
+
+
 @pytest.fixture(scope="module")
 def tiny_qwen2():
     """A qwen2-style model: neox RoPE and q/k/v biases (model.py:22-29,
