@@ -5,16 +5,18 @@
 // keeps such weights as float32 arrays, alpacca/tensor.py:91-97 multiplies
 // them with SGEMM).  Every operand enters the products exactly or in pieces:
 //   F16   W as stored (11 bits); x in two fp16 pieces after a per-row
-//         power-of-two scale (22 bits, as aq_matmul_h.hip): 2 products;
+//         power-of-two scale, the second with 2^12 more and an accumulator of
+//         its own (22 bits from 2^-28 of the row's largest on): 2 products;
 //   BF16  W as stored (8 bits); x in three bf16 pieces (24 bits): 3;
 //   F32   W and x in three bf16 pieces each: the 6 piece products of index
 //         sum at most 2 (what is dropped is below 2^-25 of a product).
 // Products are exact in fp32, the small ones of a sub-block are summed first,
-// and one accumulator runs over K.  Weights with an infinity or a NaN stay on
-// the fp32 matrix cores (aq_matmul.hip): a piece of x that is zero times an
-// infinity would be a NaN.  x may hold either: its infinities have zeros
-// for their other pieces, and against F32 weights, which have several pieces
-// themselves, the outputs of such a row are formed again in the store.
+// and one accumulator (F16: one per piece) runs over K.  Rows of X that the
+// pieces do not hold (F16: with values smaller than that; else: with an
+// infinity or a NaN) are marked, and their outputs formed again from plain fp32
+// products behind the stores.  Weights with an infinity or a NaN stay on the
+// fp32 matrix cores (aq_matmul.hip): a piece of x that is zero times an infinity
+// would be a NaN.
 //
 // One workgroup: BM rows of X, BN rows of W, stages of 64 columns of both in
 // LDS by DMA a stage ahead (rows of 128 bytes, 256 for F32, the 16-byte chunks
@@ -27,10 +29,12 @@
 // 128-row tiles also left small batches on few workgroups: 5414 x 12800 at M =
 // 2 F16 1198 -> 38 us (the weights alone: 29), F32 1311 -> 71.  What bounds it:
 // a stage's products and fragment reads (0.5 us of matrix cores in the 1.0 -
-// 1.4 us of a 128 x 128 stage), two waves per SIMD.
+// 1.4 us of a 128 x 128 stage), two waves per SIMD.  F16 with one marked row 135
+// us, with all rows marked 370 (M = 8: 26).
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "aq_internal.h"
 #include "aq_matmul_dma.h"
@@ -68,9 +72,17 @@ __device__ __forceinline__ float bf16_finite(float x) {
 
 // ---- X preparation -----------------------------------------------------------
 // One workgroup per row: NX piece planes of M x Kp 16-bit values (zeros from
-// column K to Kp), `plane` values apart.  F16: xe[m] = 15 - E for the largest
-// finite |x| = f 2^E, f in [0.5, 1) (0 without one), pieces of x 2^e; else the
-// pieces are bf16 and xe[m] = 1 for a row with an infinity or a NaN.
+// column K to Kp), `plane` values apart, and xe[m] = 2 e + (the row's outputs are
+// formed again in the store).
+//   F16: e = 15 - E for the largest finite |x| = f 2^E, f in [0.5, 1) (0 without
+//     one); hi = fp16(x 2^e), lo = fp16((x 2^e - hi) 2^12).  The products of hi
+//     and of lo have an accumulator each, so lo's own 2^12 costs nothing and
+//     every x from 2^-28 of the largest on keeps 22 bits (hi is normal from
+//     2^-14 on, and lo's last bit there is 2^-36).  Rows with a smaller x other
+//     than zero are formed again.
+//   Else the pieces are bf16 and e is 0; rows with an infinity or a NaN are
+//     formed again.
+constexpr int kLoExp = 12;
 template <int KIND>
 __global__ void __launch_bounds__(256)
     k_x_pieces(const float *__restrict__ X, int64_t K, int64_t Kp, uint16_t *__restrict__ xp,
@@ -79,23 +91,35 @@ __global__ void __launch_bounds__(256)
   const float *xr = X + m * K;
   const int t = threadIdx.x;
   int e = 0;
+  bool again = false;
   if constexpr (KIND == kF16) {
-    __shared__ float red[4];
-    float mx = 0.f;
+    __shared__ float red[2][4];
+    float mx = 0.f, mn = INFINITY;  // of the finite values, mn without zeros
+#pragma unroll 4
     for (int64_t j = 4 * (int64_t)t; j < K; j += 1024) {
       const float4 v = *reinterpret_cast<const float4 *>(xr + j);
       const float a[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mx = fmaxf(mx, __builtin_isfinite(a[i]) ? fabsf(a[i]) : 0.f);
+      for (int i = 0; i < 4; ++i) {
+        mx = fmaxf(mx, __builtin_isfinite(a[i]) ? fabsf(a[i]) : 0.f);
+        mn = fminf(mn, a[i] == 0.f ? INFINITY : fabsf(a[i]));
+      }
     }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-    if ((t & 63) == 0) red[t >> 6] = mx;
+    for (int off = 32; off > 0; off >>= 1) {
+      mx = fmaxf(mx, __shfl_xor(mx, off));
+      mn = fminf(mn, __shfl_xor(mn, off));
+    }
+    if ((t & 63) == 0) {
+      red[0][t >> 6] = mx;
+      red[1][t >> 6] = mn;
+    }
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    mn = fminf(fminf(red[1][0], red[1][1]), fminf(red[1][2], red[1][3]));
     e = mx > 0.f ? 15 - __builtin_amdgcn_frexp_expf(mx) : 0;
+    again = __builtin_amdgcn_ldexpf(mn, e) < 0x1p-14f;
   }
-  bool bad = false;
   for (int64_t j = 4 * (int64_t)t; j < Kp; j += 1024) {
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (j < K) v = *reinterpret_cast<const float4 *>(xr + j);
@@ -103,7 +127,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if constexpr (KIND == kF16) a[i] = __builtin_amdgcn_ldexpf(a[i], e);
-      else bad = bad || !__builtin_isfinite(a[i]);
+      else again = again || !__builtin_isfinite(a[i]);
     }
 #pragma unroll
     for (int p = 0; p < pieces_of(KIND); ++p) {
@@ -113,8 +137,8 @@ __global__ void __launch_bounds__(256)
         float &x = a[2 * i], &y = a[2 * i + 1];
         if constexpr (KIND == kF16) {
           w[i] = pack_f16(x, y);
-          x = rest_of(x, (float)(_Float16)x);
-          y = rest_of(y, (float)(_Float16)y);
+          x = rest_of(x, (float)(_Float16)x) * (float)(1 << kLoExp);
+          y = rest_of(y, (float)(_Float16)y) * (float)(1 << kLoExp);
         } else {
           w[i] = pack_bf16(bf16_finite(x), bf16_finite(y));
           x = rest_of(x, __uint_as_float(w[i] << 16));
@@ -124,8 +148,8 @@ __global__ void __launch_bounds__(256)
       *reinterpret_cast<uint2 *>(xp + p * plane + m * Kp + j) = make_uint2(w[0], w[1]);
     }
   }
-  if constexpr (KIND != kF16) e = __syncthreads_or(bad) ? 1 : 0;
-  if (t == 0) xe[m] = e;
+  if constexpr (KIND != kF16) again = __syncthreads_or(again);
+  if (t == 0) xe[m] = 2 * e + (again ? 1 : 0);
 }
 
 // ---- tile kernel -----------------------------------------------------------------
@@ -146,6 +170,63 @@ __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a),
                                                    __builtin_bit_cast(b8, b), c, 0, 0, 0);
+}
+
+// NT tiles of plain fp32 products over columns k_begin .. k_end (a multiple of
+// 32 long, not none): 16 rows of X (this lane's: `row`) by 16 rows of W each
+// (this lane's of tile j: n + 16 j, row N - 1 past the last).  Lane group g takes
+// columns 4 g .. +3 of every 16; the next 32 columns are loaded during the
+// products of these.
+template <int KIND, int NT>
+__device__ __forceinline__ void plain_tile(const float *X, int64_t row, const uint8_t *W, int64_t n,
+                                           int64_t N, int64_t K, int64_t k_begin, int64_t k_end,
+                                           int g, f32x4 (&o)[NT]) {
+  constexpr int ESZ = KIND == kF32 ? 4 : 2;
+  using Raw = std::conditional_t<KIND == kF32, f32x4, uint2>;  // four weights
+  const float *xr = X + row * K + 4 * g;
+  const uint8_t *wr[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    wr[j] = W + ((n + 16 * j < N ? n + 16 * j : N - 1) * K + 4 * g) * ESZ;
+    o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  f32x4 x[2], xn[2];
+  Raw w[2][NT], wn[2][NT];
+  auto load = [&](int64_t k, f32x4 (&xd)[2], Raw (&wd)[2][NT]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      xd[h] = *reinterpret_cast<const f32x4 *>(xr + k + 16 * h);
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        wd[h][j] = *reinterpret_cast<const Raw *>(wr[j] + (k + 16 * h) * ESZ);
+    }
+  };
+  load(k_begin, x, w);
+  for (int64_t k = k_begin; k < k_end; k += 32) {
+    load(k + 32 < k_end ? k + 32 : k, xn, wn);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          float v;
+          if constexpr (KIND == kF32) {
+            v = w[h][j][t];
+          } else {
+            const uint32_t b = (t < 2 ? w[h][j].x : w[h][j].y) >> (16 * (t & 1)) & 0xFFFFu;
+            v = KIND == kF16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)b)
+                             : __uint_as_float(b << 16);
+          }
+          o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[h][t], v, o[j], 0, 0, 0);
+        }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      x[h] = xn[h];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) w[h][j] = wn[h][j];
+    }
+  }
 }
 
 template <int KIND, int MT, int NT, int WGM, int WGN>
@@ -175,7 +256,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
   // X stage: NX x BM rows of 128 bytes, chunk c of row r in slot c ^ (r & 7);
   // rows past M repeat row M - 1
   constexpr int XI = NX * BM / 8 / WAVES, XP = BM / 8, XR = XP / WAVES;
-  static_assert(XP % WAVES == 0, "whole DMAs per wave and piece");
+  static_assert(XP % WAVES == 0 && MT * 16 <= 64, "whole DMAs per wave and piece; a lane per row");
   uint32_t vx[XR];
 #pragma unroll
   for (int i = 0; i < XR; ++i) {
@@ -245,16 +326,25 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
     }
   };
 
-  f32x4 acc[MT][NT];
+  // F16: acc[0] takes the products of hi, acc[1] those of lo
+  constexpr int NA = KIND == kF16 ? 2 : 1;
+  f32x4 acc[NA][MT][NT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int a = 0; a < NA; ++a)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[a][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // A fragments are read two steps ahead (ring A), B a sub-block ahead.  At
   // step STEPS - 2 of a stage's second sub-block every fragment of the stage
   // is in registers: the barrier there publishes the next stage, issued a
   // stage ago, and frees this one's buffer.
   u32x4 A[4], B[2][NT][NB];
+  // exponents and marks of the wave's rows, row i in lane i: loaded here and pinned
+  // behind a stage's barrier (in the stores their latency would be 0.3 us of every
+  // call)
+  const int64_t my_row = m0 + wm * MT * 16 + lane;
+  int mark = lane < MT * 16 && my_row < M ? xe[my_row] : 0;
   dma_stage(s_begin, 0);
   if (s_begin + 1 < s_end) {
     dma_stage(s_begin + 1, 1);
@@ -275,6 +365,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
         const int step = e * STEPS + k;
         if (e == 1 && k == STEPS - 2 && st + 1 < s_end) {
           dma_barrier<0>();
+          asm volatile("" : "+v"(mark));
           if (st + 2 < s_end) dma_stage(st + 2, buf);
         }
         // (past the last stage: whatever the other buffer holds, not used)
@@ -287,7 +378,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
         for (int q = NB - 1; q >= 0; --q)
 #pragma unroll
           for (int j = 0; j < NT; ++j)
-            if (p + q <= 2) acc[i][j] = mfma<KIND>(A[step % 4], B[e][j][q], acc[i][j]);
+            if (p + q <= 2)
+              acc[p % NA][i][j] = mfma<KIND>(A[step % 4], B[e][j][q], acc[p % NA][i][j]);
         if (e == 0) {
 #pragma unroll
           for (int j = k * NT / STEPS; j < (k + 1) * NT / STEPS; ++j) read_b(buf, 1, j, B[1][j]);
@@ -304,25 +396,43 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
       const int64_t row = m0 + (wm * MT + i) * 16 + 4 * g + rr;
+      int ex = 0;
+      if constexpr (KIND == kF16) ex = __shfl(mark, i * 16 + 4 * g + rr) >> 1;
       if (row >= M) continue;
-      const int ex = xe[row];
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const int64_t n = n0 + (wn * NT + j) * 16 + c16;
         if (n >= N) continue;
-        float v = acc[i][j][rr];
-        if constexpr (KIND == kF16) v = __builtin_amdgcn_ldexpf(v, -ex);
-        if constexpr (KIND == kF32) {
-          if (ex) {  // the row's plain fp32 sum, from the first split alone
-            const float *wr = reinterpret_cast<const float *>(W) + n * K;
-            v = 0.f;
-            if (blockIdx.z == 0)
-              for (int64_t k = 0; k < K; ++k) v = fmaf(X[row * K + k], wr[k], v);
-          }
-        }
+        float v = acc[0][i][j][rr];
+        if constexpr (KIND == kF16)
+          v = __builtin_amdgcn_ldexpf(fmaf(acc[NA - 1][i][j][rr], 1.f / (1 << kLoExp), v), -ex);
         Y[row * N + n] = v;
       }
     }
+  // Marked rows again, over what was stored (at the end: code that the stores
+  // jump over costs every call 0.5 us of instruction fetches)
+  if (__builtin_expect(__any(mark & 1), 0)) {
+    const int64_t k_begin = 64 * (int64_t)s_begin, k_end = std::min(64 * (int64_t)s_end, K);
+#pragma unroll 1
+    for (int i = 0; i < MT; ++i) {
+      const int64_t row0 = m0 + (wm * MT + i) * 16;
+      bool redo[4];
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr)  // (rows past M have no mark)
+        redo[rr] = __shfl(mark, i * 16 + 4 * g + rr) & 1;
+      if (!__any(redo[0] || redo[1] || redo[2] || redo[3])) continue;
+      f32x4 plain[NT];
+      plain_tile<KIND, NT>(X, row0 + c16 < M ? row0 + c16 : M - 1, W, n0 + wn * NT * 16 + c16, N, K,
+                           k_begin, k_end, g, plain);
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const int64_t n = n0 + (wn * NT + j) * 16 + c16;
+          if (redo[rr] && n < N) Y[(row0 + 4 * g + rr) * N + n] = plain[j][rr];
+        }
+    }
+  }
 }
 
 struct DnLaunch {

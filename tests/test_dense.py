@@ -188,9 +188,12 @@ def test_dense_tile_shapes_vs_f64(dtype, M, rows, cols, monkeypatch):
 @pytest.mark.parametrize("dtype", DENSE)
 def test_dense_matmul_t_nonfinite(dtype):
     """Infinities and NaNs in X and in the weights give what float32 products
-    give, and leave the other rows and columns alone."""
+    give, and leave the other rows and columns alone.  Bar: the rounding of a sum
+    of cols float32 products, cols 2^-24 of the sum of |x| |w|, for each output
+    (weights of zero against the largest x leave the rest of its row's sum)."""
     M, rows, cols = 40, 64, 128
     w = np.random.default_rng(1).standard_normal((rows, cols)).astype(np.float32)
+    w[20:40, 8] = 0.0
     if dtype == "BF16":
         w = (w.view(np.uint32) & 0xFFFF0000).view(np.float32)
     X = synth.random_x(cols, seed=2, batch=M)
@@ -209,8 +212,54 @@ def test_dense_matmul_t_nonfinite(dtype):
         fin = np.isfinite(want)
         assert np.array_equal(np.isnan(want), np.isnan(Y))
         assert np.array_equal(want[~fin & ~np.isnan(want)], Y[~fin & ~np.isnan(want)])
-        scale = np.abs(X).max(axis=1, keepdims=True) * 64
-        assert (np.abs(Y - want)[fin] < 1e-5 * np.broadcast_to(scale, Y.shape)[fin]).all()
+        with np.errstate(invalid="ignore"):
+            bar = (np.abs(X).astype(np.float64) @ np.abs(wv).T) * cols * 2.0 ** -24
+        assert (np.abs(Y[fin].astype(np.float64) - want[fin]) <= bar[fin]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DENSE)
+@pytest.mark.parametrize("cols", [64, 2080])
+def test_dense_matmul_t_wide_range_rows(dtype, cols, monkeypatch):
+    """Rows of X whose elements lie far apart: what is left of a sum when the
+    weight of the largest element is zero has the accuracy of float32 products.
+    Bar: cols 2^-24 of the sum of |x| |w|, for each output.  F16 keeps 22 bits of
+    elements down to 2^-28 of the row's largest in its two pieces (row 0) and
+    forms rows with smaller ones again in float32; one row of each kind per
+    16-row tile, with a split of K (auto, 2080 columns) and without, the same
+    bits in every tile shape at fp32."""
+    M, rows = 37, 150
+    rng = np.random.default_rng(cols)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    w = (w.view(np.uint32) & 0xFFFF0000).view(np.float32)
+    w[:, 7] = 0.0
+    data = (w.astype(np.float16).view(np.uint8) if dtype == "F16" else
+            (w.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8) if dtype == "BF16"
+            else w.view(np.uint8)).reshape(-1)
+    wv = w.astype(np.float16).astype(np.float64) if dtype == "F16" else w.astype(np.float64)
+    X = synth.random_x(cols, seed=cols, batch=M)
+    X[0] = rng.uniform(0.5, 1.0, cols) * rng.choice([-1.0, 1.0], cols)
+    X[0, 7] = 2.0 ** 27
+    X[17, 7] = 1e8
+    X[18] = 1.0
+    X[18, 7] = 1e20
+    X[35] = np.ldexp(X[35], rng.integers(-90, 90, cols))
+    X[36] = 0.0
+    X[36, 7], X[36, 9] = 3e38, 1e-30
+    want = X.astype(np.float64) @ wv.T
+    bar = (np.abs(X).astype(np.float64) @ np.abs(wv).T) * cols * 2.0 ** -24
+    W = DenseMatrix(data, dtype, rows, cols)
+    first = None
+    for shape in (None, 0, 1, 2, 3):
+        if shape is not None:
+            monkeypatch.setenv("AQ_MATMUL_TILE", str(shape))
+        for prec in ("auto", "fp32"):
+            Y = W.matmul_t(X, precision=prec)
+            bad = np.argwhere(np.abs(Y.astype(np.float64) - want) > bar)
+            assert not len(bad), (shape, prec, bad[:5])
+            if prec == "fp32":
+                first = Y if first is None else first
+                assert np.array_equal(Y.view(np.uint32), first.view(np.uint32)), shape
 
 
 @pytest.mark.gpu
