@@ -11,10 +11,10 @@
 //   F32   W and x in three bf16 pieces each: the 6 piece products of index
 //         sum at most 2 (what is dropped is below 2^-25 of a product).
 // Products are exact in fp32, the small ones of a sub-block are summed first,
-// and one accumulator (F16: one per piece) runs over K.  Rows of X that the
-// pieces do not hold (F16: with values smaller than that; else: with an
-// infinity or a NaN) are marked, and their outputs formed again from plain fp32
-// products behind the stores.  Weights with an infinity or a NaN stay on the
+// and one accumulator (F16: one per piece) runs over K.  Behind the stores,
+// what the pieces of a row lack is added (F16: up to eight values below that
+// range), or the row's outputs are formed again from plain fp32 products (more
+// of them; else: rows with an infinity or a NaN).  Weights with an infinity or a NaN stay on the
 // fp32 matrix cores (aq_matmul.hip): a piece of x that is zero times an infinity
 // would be a NaN.
 //
@@ -29,8 +29,10 @@
 // 128-row tiles also left small batches on few workgroups: 5414 x 12800 at M =
 // 2 F16 1198 -> 38 us (the weights alone: 29), F32 1311 -> 71.  What bounds it:
 // a stage's products and fragment reads (0.5 us of matrix cores in the 1.0 -
-// 1.4 us of a 128 x 128 stage), two waves per SIMD.  F16 with one marked row 135
-// us, with all rows marked 370 (M = 8: 26).
+// 1.4 us of a 128 x 128 stage), two waves per SIMD.  F16 rows with values below
+// the pieces' range, 4096 x 14336 at M = 512, 141 us for normal ones: SwiGLU
+// outputs (0.7 % of rows have one) 143, every row with a few 203, every row
+// formed again 1264 (the fp32 kernel: 919).
 #include <stdlib.h>
 
 #include <algorithm>
@@ -72,28 +74,37 @@ __device__ __forceinline__ float bf16_finite(float x) {
 
 // ---- X preparation -----------------------------------------------------------
 // One workgroup per row: NX piece planes of M x Kp 16-bit values (zeros from
-// column K to Kp), `plane` values apart, and xe[m] = 2 e + (the row's outputs are
-// formed again in the store).
+// column K to Kp), `plane` values apart, and xe[m] = 16 e + mark.
 //   F16: e = 15 - E for the largest finite |x| = f 2^E, f in [0.5, 1) (0 without
 //     one); hi = fp16(x 2^e), lo = fp16((x 2^e - hi) 2^12).  The products of hi
 //     and of lo have an accumulator each, so lo's own 2^12 costs nothing and
 //     every x from 2^-28 of the largest on keeps 22 bits (hi is normal from
-//     2^-14 on, and lo's last bit there is 2^-36).  Rows with a smaller x other
-//     than zero are formed again.
-//   Else the pieces are bf16 and e is 0; rows with an infinity or a NaN are
-//     formed again.
-constexpr int kLoExp = 12;
+//     2^-14 on, and lo's last bit there is 2^-36).  What the pieces lack of
+//     smaller values other than zero is listed, xl[m] (a row of SwiGLU outputs
+//     14,336 wide has one in 0.7 % of cases): mark = entries, or kAgain for more
+//     than kList of them.
+//   Else the pieces are bf16, e is 0 and the mark of rows with an infinity or a
+//     NaN kAgain.
+// Marked rows are corrected, or formed again, after the stores.
+constexpr int kLoExp = 12, kList = 8, kAgain = 15;
+struct Lacking {
+  int32_t k;
+  float x;
+};
 template <int KIND>
 __global__ void __launch_bounds__(256)
     k_x_pieces(const float *__restrict__ X, int64_t K, int64_t Kp, uint16_t *__restrict__ xp,
-               int64_t plane, int32_t *__restrict__ xe) {
+               int64_t plane, int32_t *__restrict__ xe, Lacking *__restrict__ xl) {
   const int64_t m = blockIdx.x;
   const float *xr = X + m * K;
   const int t = threadIdx.x;
   int e = 0;
-  bool again = false;
+  bool again = false;  // F16: some of the row's values are to be listed
+  __shared__ int n_list;
+  __shared__ Lacking list[kList];
   if constexpr (KIND == kF16) {
     __shared__ float red[2][4];
+    if (t == 0) n_list = 0;
     float mx = 0.f, mn = INFINITY;  // of the finite values, mn without zeros
 #pragma unroll 4
     for (int64_t j = 4 * (int64_t)t; j < K; j += 1024) {
@@ -124,6 +135,19 @@ __global__ void __launch_bounds__(256)
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (j < K) v = *reinterpret_cast<const float4 *>(xr + j);
     float a[4] = {v.x, v.y, v.z, v.w};
+    if (KIND == kF16 && again)
+      for (int i = 0; i < 4; ++i) {
+        const float x = i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
+        const float y = __builtin_amdgcn_ldexpf(x, e);
+        if (x == 0.f || !(fabsf(y) < 0x1p-14f)) continue;
+        const float hi = (float)(_Float16)y;
+        const float lo = (float)(_Float16)((y - hi) * (1 << kLoExp));
+        // (exact: the pieces hold 22 bits next to x's own)
+        const float d = x - __builtin_amdgcn_ldexpf(fmaf(lo, 1.f / (1 << kLoExp), hi), -e);
+        if (d == 0.f) continue;
+        const int slot = atomicAdd(&n_list, 1);
+        if (slot < kList) list[slot] = Lacking{(int32_t)j + i, d};
+      }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if constexpr (KIND == kF16) a[i] = __builtin_amdgcn_ldexpf(a[i], e);
@@ -148,8 +172,19 @@ __global__ void __launch_bounds__(256)
       *reinterpret_cast<uint2 *>(xp + p * plane + m * Kp + j) = make_uint2(w[0], w[1]);
     }
   }
-  if constexpr (KIND != kF16) again = __syncthreads_or(again);
-  if (t == 0) xe[m] = 2 * e + (again ? 1 : 0);
+  int mark = 0;
+  if constexpr (KIND != kF16) {
+    mark = __syncthreads_or(again) ? kAgain : 0;
+  } else if (again) {  // the same for the whole workgroup
+    __syncthreads();
+    mark = n_list <= kList ? n_list : kAgain;
+    if (t < mark && mark <= kList) {  // in column order
+      int at = 0;
+      for (int i = 0; i < mark; ++i) at += list[i].k < list[t].k;
+      xl[m * kList + at] = list[t];
+    }
+  }
+  if (t == 0) xe[m] = 16 * e + mark;
 }
 
 // ---- tile kernel -----------------------------------------------------------------
@@ -232,8 +267,8 @@ __device__ __forceinline__ void plain_tile(const float *X, int64_t row, const ui
 template <int KIND, int MT, int NT, int WGM, int WGN>
 __global__ void __launch_bounds__(64 * WGM * WGN)
     k_mm_dn(const uint8_t *W, int64_t N, int64_t K, const uint16_t *xp, int64_t plane, int64_t Kp,
-            const int32_t *__restrict__ xe, const float *__restrict__ X, int64_t M,
-            float *__restrict__ Y, int per_split, int m_tiles, int n_tiles) {
+            const int32_t *__restrict__ xe, const Lacking *__restrict__ xl,
+            const float *__restrict__ X, int64_t M, float *__restrict__ Y, int per_split, int m_tiles, int n_tiles) {
   using T = DnTile<KIND, MT, NT, WGM, WGN>;
   constexpr int BM = T::BM, BN = T::BN, WAVES = T::kWaves, NX = pieces_of(KIND);
   constexpr int NB = KIND == kF32 ? 3 : 1;           // pieces of W
@@ -397,7 +432,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
     for (int rr = 0; rr < 4; ++rr) {
       const int64_t row = m0 + (wm * MT + i) * 16 + 4 * g + rr;
       int ex = 0;
-      if constexpr (KIND == kF16) ex = __shfl(mark, i * 16 + 4 * g + rr) >> 1;
+      if constexpr (KIND == kF16) ex = __shfl(mark, i * 16 + 4 * g + rr) >> 4;
       if (row >= M) continue;
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
@@ -409,18 +444,37 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
         Y[row * N + n] = v;
       }
     }
-  // Marked rows again, over what was stored (at the end: code that the stores
-  // jump over costs every call 0.5 us of instruction fetches)
-  if (__builtin_expect(__any(mark & 1), 0)) {
+  // Marked rows, over what was stored (at the end: code that the stores jump over
+  // costs every call 0.5 us of instruction fetches)
+  if (__builtin_expect(__any(mark & 15), 0)) {
     const int64_t k_begin = 64 * (int64_t)s_begin, k_end = std::min(64 * (int64_t)s_end, K);
 #pragma unroll 1
     for (int i = 0; i < MT; ++i) {
       const int64_t row0 = m0 + (wm * MT + i) * 16;
-      bool redo[4];
+      int todo[4];
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr)  // (rows past M have no mark)
-        redo[rr] = __shfl(mark, i * 16 + 4 * g + rr) & 1;
-      if (!__any(redo[0] || redo[1] || redo[2] || redo[3])) continue;
+        todo[rr] = __shfl(mark, i * 16 + 4 * g + rr) & 15;
+      if constexpr (KIND == kF16) {
+#pragma unroll 1
+        for (int rr = 0; rr < 4; ++rr) {
+          const int64_t row = row0 + 4 * g + rr;
+          const int count = todo[rr] == kAgain ? 0 : todo[rr];
+#pragma unroll 1
+          for (int c = 0; c < count; ++c) {
+            const Lacking l = xl[row * kList + c];
+            if (l.k < k_begin || l.k >= k_end) continue;  // another split's
+            for (int j = 0; j < NT; ++j) {
+              const int64_t n = n0 + (wn * NT + j) * 16 + c16;
+              if (n < N)
+                Y[row * N + n] = fmaf(l.x, (float)reinterpret_cast<const _Float16 *>(W)[n * K + l.k],
+                                      Y[row * N + n]);
+            }
+          }
+        }
+      }
+      if (!__any(todo[0] == kAgain || todo[1] == kAgain || todo[2] == kAgain || todo[3] == kAgain))
+        continue;
       f32x4 plain[NT];
       plain_tile<KIND, NT>(X, row0 + c16 < M ? row0 + c16 : M - 1, W, n0 + wn * NT * 16 + c16, N, K,
                            k_begin, k_end, g, plain);
@@ -429,7 +483,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
           const int64_t n = n0 + (wn * NT + j) * 16 + c16;
-          if (redo[rr] && n < N) Y[(row0 + 4 * g + rr) * N + n] = plain[j][rr];
+          if (todo[rr] == kAgain && n < N) Y[(row0 + 4 * g + rr) * N + n] = plain[j][rr];
         }
     }
   }
@@ -440,6 +494,7 @@ struct DnLaunch {
   const uint16_t *xp;
   int64_t plane, Kp;
   const int32_t *xe;
+  const Lacking *xl;
   const float *X;
   int64_t M;
   float *dst;
@@ -454,7 +509,7 @@ hipError_t launch_tile(const DnLaunch &a) {
   auto kern = k_mm_dn<KIND, MT, NT, WGM, WGN>;
   if (hipError_t e = set_dynamic_lds(reinterpret_cast<const void *>(kern), T::kLds)) return e;
   hipLaunchKernelGGL(kern, grid, dim3(T::kThreads), T::kLds, a.s, a.m->planes.p[0], a.m->rows,
-                     a.m->cols, a.xp, a.plane, a.Kp, a.xe, a.X, a.M, a.dst, a.per, mt, nt);
+                     a.m->cols, a.xp, a.plane, a.Kp, a.xe, a.xl, a.X, a.M, a.dst, a.per, mt, nt);
   return hipGetLastError();
 }
 template <int KIND>
@@ -543,22 +598,24 @@ hipError_t launch_matmul_dn(const aq_matrix *m, const float *X, int64_t M, float
   splits = (units + per - 1) / per;
   auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
   const int64_t plane = M * Kp;
-  const size_t xb = al((size_t)pieces_of(kind) * plane * 2), eb = al((size_t)M * 4);
+  const size_t xb = al((size_t)pieces_of(kind) * plane * 2), eb = al((size_t)M * 4),
+               lb = kind == kF16 ? al((size_t)M * kList * sizeof(Lacking)) : 0;
   const size_t part = splits > 1 ? (size_t)splits * M * N * 4 : 0;
-  uint8_t *ws = static_cast<uint8_t *>(workspace(m->device, s, xb + eb + part));
+  uint8_t *ws = static_cast<uint8_t *>(workspace(m->device, s, xb + eb + lb + part));
   if (!ws) {
     *no_scratch = true;
     return hipErrorOutOfMemory;
   }
   uint16_t *xp = reinterpret_cast<uint16_t *>(ws);
   int32_t *xe = reinterpret_cast<int32_t *>(ws + xb);
-  float *dst = splits > 1 ? reinterpret_cast<float *>(ws + xb + eb) : Y;
+  Lacking *xl = reinterpret_cast<Lacking *>(ws + xb + eb);
+  float *dst = splits > 1 ? reinterpret_cast<float *>(ws + xb + eb + lb) : Y;
 #define AQ_XP(k) \
-  hipLaunchKernelGGL(k_x_pieces<k>, dim3((unsigned)M), dim3(256), 0, s, X, K, Kp, xp, plane, xe)
+  hipLaunchKernelGGL(k_x_pieces<k>, dim3((unsigned)M), dim3(256), 0, s, X, K, Kp, xp, plane, xe, xl)
   if (kind == kF16) AQ_XP(kF16);
   else AQ_XP(kBF16);  // (the same pieces for F32)
 #undef AQ_XP
-  const DnLaunch a{m, xp, plane, Kp, xe, X, M, dst, splits, per, s};
+  const DnLaunch a{m, xp, plane, Kp, xe, xl, X, M, dst, splits, per, s};
   const hipError_t e = kind == kF16    ? launch_shape<kF16>(shape, a)
                        : kind == kBF16 ? launch_shape<kBF16>(shape, a)
                                        : launch_shape<kF32>(shape, a);

@@ -224,28 +224,35 @@ def test_dense_matmul_t_wide_range_rows(dtype, cols, monkeypatch):
     """Rows of X whose elements lie far apart: what is left of a sum when the
     weight of the largest element is zero has the accuracy of float32 products.
     Bar: cols 2^-24 of the sum of |x| |w|, for each output.  F16 keeps 22 bits of
-    elements down to 2^-28 of the row's largest in its two pieces (row 0) and
-    forms rows with smaller ones again in float32; one row of each kind per
-    16-row tile, with a split of K (auto, 2080 columns) and without, the same
-    bits in every tile shape at fp32."""
+    elements down to 2^-28 of the row's largest in its two pieces (row 0), adds
+    what they lack of up to eight smaller ones (rows 1 - 3: one, eight, and nine
+    of them, the last is formed again in float32 as rows 17, 18, 35 are); with
+    a split of K (auto, 2080 columns) and without, the same bits in every tile
+    shape at fp32."""
     M, rows = 37, 150
     rng = np.random.default_rng(cols)
     w = rng.standard_normal((rows, cols)).astype(np.float32)
     w = (w.view(np.uint32) & 0xFFFF0000).view(np.float32)
     w[:, 7] = 0.0
-    data = (w.astype(np.float16).view(np.uint8) if dtype == "F16" else
-            (w.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8) if dtype == "BF16"
-            else w.view(np.uint8)).reshape(-1)
-    wv = w.astype(np.float16).astype(np.float64) if dtype == "F16" else w.astype(np.float64)
     X = synth.random_x(cols, seed=cols, batch=M)
     X[0] = rng.uniform(0.5, 1.0, cols) * rng.choice([-1.0, 1.0], cols)
     X[0, 7] = 2.0 ** 27
+    for i, n in ((1, 1), (2, 8), (3, 9)):
+        # small values against weights of 2^13, so that the sum shows them
+        X[i] = rng.uniform(0.5, 1.0, cols) * rng.choice([-1.0, 1.0], cols)
+        X[i, 7], X[i, 8:] = 2.0 ** 27, 0.0
+        X[i, cols - 3 * n::3] = rng.uniform(1.0, 2.0, n) * 2.0 ** -21
+    w[::2, cols - 40:] *= np.float32(2.0 ** 13)
     X[17, 7] = 1e8
     X[18] = 1.0
     X[18, 7] = 1e20
     X[35] = np.ldexp(X[35], rng.integers(-90, 90, cols))
     X[36] = 0.0
     X[36, 7], X[36, 9] = 3e38, 1e-30
+    data = (w.astype(np.float16).view(np.uint8) if dtype == "F16" else
+            (w.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8) if dtype == "BF16"
+            else w.view(np.uint8)).reshape(-1)
+    wv = w.astype(np.float16).astype(np.float64) if dtype == "F16" else w.astype(np.float64)
     want = X.astype(np.float64) @ wv.T
     bar = (np.abs(X).astype(np.float64) @ np.abs(wv).T) * cols * 2.0 ** -24
     W = DenseMatrix(data, dtype, rows, cols)
