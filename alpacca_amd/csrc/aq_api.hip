@@ -599,9 +599,9 @@ int aq_matrix_create(const void *blocks, size_t nbytes, int dtype, int64_t rows,
     delete m;
     return hip_fail(e, "hipMemcpy(matrix upload)");
   }
-  m->finite = true;
+  m->in_range = true;
   if (aq::is_dense(dtype)) {
-    e = aq::dense_all_finite(m, &m->finite);
+    e = aq::dense_in_range(m, &m->in_range);
     if (e != hipSuccess) {
       (void)hipFree(m->dev);
       delete m;

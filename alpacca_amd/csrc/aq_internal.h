@@ -23,7 +23,7 @@ struct aq_matrix {
   uint8_t *dev;         // one hipMalloc holding every plane
   size_t dev_bytes;
   aq::Planes planes;
-  bool finite;          // dense: no infinity or NaN among the weights
+  bool in_range;        // dense: weights that aq_matmul_dn.hip takes (dense_in_range)
 };
 
 namespace aq {
@@ -82,12 +82,13 @@ hipError_t launch_matmul_h(const aq_matrix *m, const float *X, int64_t M, float 
                            bool *fused_sw = nullptr);
 
 // matmul_t of dense weights on 16-bit matrix cores at float32 accuracy
-// (aq_matmul_dn.hip), for matrices without infinities and NaNs
-// (mm_dn_supported; dense_all_finite looks through a matrix's device copy).
+// (aq_matmul_dn.hip), for matrices without infinities, NaNs and (F32) values
+// that three bf16 pieces do not hold (mm_dn_supported; dense_in_range looks
+// through a matrix's device copy).
 // m_invariant as for launch_matmul_h.  *no_scratch: nothing was launched, since
 // the stream's workspace cannot hold the pieces of X.
 bool mm_dn_supported(const aq_matrix *m);
-hipError_t dense_all_finite(const aq_matrix *m, bool *finite);
+hipError_t dense_in_range(const aq_matrix *m, bool *in_range);
 hipError_t launch_matmul_dn(const aq_matrix *m, const float *X, int64_t M, float *Y,
                             bool m_invariant, hipStream_t s, bool *no_scratch);
 // Takes back the notes of a refused workspace (a capture's, HIP's last

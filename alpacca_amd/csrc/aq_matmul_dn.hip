@@ -14,9 +14,10 @@
 // and one accumulator (F16: one per piece) runs over K.  Behind the stores,
 // what the pieces of a row lack is added (F16: up to eight values below that
 // range), or the row's outputs are formed again from plain fp32 products (more
-// of them; else: rows with an infinity or a NaN).  Weights with an infinity or a NaN stay on the
-// fp32 matrix cores (aq_matmul.hip): a piece of x that is zero times an infinity
-// would be a NaN.
+// of them; else: rows with an infinity, a NaN or a value below 2^-110).  Weights
+// with an infinity or a NaN, and F32 weights below 2^-110, stay on the fp32
+// matrix cores (aq_matmul.hip): a piece of x that is zero times an infinity
+// would be a NaN, and three pieces hold 24 bits from 2^-110 on.
 //
 // One workgroup: BM rows of X, BN rows of W, stages of 64 columns of both in
 // LDS by DMA a stage ahead (rows of 128 bytes, 256 for F32, the 16-byte chunks
@@ -83,9 +84,12 @@ __device__ __forceinline__ float bf16_finite(float x) {
 //     smaller values other than zero is listed, xl[m] (a row of SwiGLU outputs
 //     14,336 wide has one in 0.7 % of cases): mark = entries, or kAgain for more
 //     than kList of them.
-//   Else the pieces are bf16, e is 0 and the mark of rows with an infinity or a
-//     NaN kAgain.
+//   Else the pieces are bf16, e is 0 and the mark of rows with an infinity, a NaN
+//     or a value below kPieceMin other than zero kAgain.
 // Marked rows are corrected, or formed again, after the stores.
+// the smallest magnitude whose 24 bits three bf16 pieces hold: its last bit is
+// bf16's smallest subnormal, 2^-133 (the matrix cores keep subnormal inputs)
+constexpr float kPieceMin = 0x1p-110f;
 constexpr int kLoExp = 12, kList = 8, kAgain = 15;
 struct Lacking {
   int32_t k;
@@ -151,7 +155,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if constexpr (KIND == kF16) a[i] = __builtin_amdgcn_ldexpf(a[i], e);
-      else again = again || !__builtin_isfinite(a[i]);
+      else again = again || !__builtin_isfinite(a[i]) || (a[i] != 0.f && fabsf(a[i]) < kPieceMin);
     }
 #pragma unroll
     for (int p = 0; p < pieces_of(KIND); ++p) {
@@ -536,18 +540,21 @@ constexpr TileCost kTiles[] = {
 constexpr int kTileShapes = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr TileModel kModel = {kTiles, kTileShapes, 1.f, 1.f / 3.6f};
 
-// A value among n 16- or 32-bit ones with an exponent field of at least `low`
+// A value among n 16- or 32-bit ones with a magnitude (as its bits) of at least
+// `high`, or below `low` and not zero
 template <class W>
-__global__ void k_nonfinite(const W *__restrict__ p, int64_t n, W mask, W low, int *flag) {
+__global__ void k_out_of_range(const W *__restrict__ p, int64_t n, W low, W high, int *flag) {
   bool bad = false;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-    bad = bad || (p[i] & mask) >= low;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const W u = p[i] & (W)((W)~(W)0 >> 1);
+    bad = bad || u >= high || (u != 0 && u < low);
+  }
   if (bad) *flag = 1;
 }
 }  // namespace
 
-hipError_t dense_all_finite(const aq_matrix *m, bool *finite) {
-  *finite = true;
+hipError_t dense_in_range(const aq_matrix *m, bool *in_range) {
+  *in_range = true;
   const int64_t n = m->rows * m->cols;
   if (n == 0) return hipSuccess;
   int *flag = nullptr, host = 0;
@@ -556,26 +563,25 @@ hipError_t dense_all_finite(const aq_matrix *m, bool *finite) {
   e = hipMemcpy(flag, &host, sizeof(int), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     const unsigned wg = (unsigned)std::min<int64_t>((n + 255) / 256, 4096);
-    if (m->dtype == AQ_F32)
-      hipLaunchKernelGGL((k_nonfinite<uint32_t>), dim3(wg), dim3(256), 0, nullptr,
-                         reinterpret_cast<const uint32_t *>(m->planes.p[0]), n, 0x7F800000u,
-                         0x7F000000u, flag);  // (from 2^127 on a bf16 piece may round to infinity)
+    if (m->dtype == AQ_F32)  // (from 2^127 on a bf16 piece may round to infinity)
+      hipLaunchKernelGGL((k_out_of_range<uint32_t>), dim3(wg), dim3(256), 0, nullptr,
+                         reinterpret_cast<const uint32_t *>(m->planes.p[0]), n,
+                         __builtin_bit_cast(uint32_t, kPieceMin), 0x7F000000u, flag);
     else
-      hipLaunchKernelGGL((k_nonfinite<uint16_t>), dim3(wg), dim3(256), 0, nullptr,
-                         reinterpret_cast<const uint16_t *>(m->planes.p[0]), n,
-                         (uint16_t)(m->dtype == AQ_F16 ? 0x7C00u : 0x7F80u),
+      hipLaunchKernelGGL((k_out_of_range<uint16_t>), dim3(wg), dim3(256), 0, nullptr,
+                         reinterpret_cast<const uint16_t *>(m->planes.p[0]), n, (uint16_t)0,
                          (uint16_t)(m->dtype == AQ_F16 ? 0x7C00u : 0x7F80u), flag);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpy(&host, flag, sizeof(int), hipMemcpyDeviceToHost);
   (void)hipFree(flag);
-  *finite = host == 0;
+  *in_range = host == 0;
   return e;
 }
 
 bool mm_dn_supported(const aq_matrix *m) {
   // 32-bit offsets into W
-  return is_dense(m->dtype) && m->finite && m->nb_pitch == m->nb_row && m->cols > 0 &&
+  return is_dense(m->dtype) && m->in_range && m->nb_pitch == m->nb_row && m->cols > 0 &&
          (double)m->rows * (double)m->cols * (m->dtype == AQ_F32 ? 4.0 : 2.0) < 4294967296.0;
 }
 

@@ -269,6 +269,51 @@ def test_dense_matmul_t_wide_range_rows(dtype, cols, monkeypatch):
                 assert np.array_equal(Y.view(np.uint32), first.view(np.uint32)), shape
 
 
+def _f64_of_bits(x):
+    """float32 values as float64 from their bits (a process in which some library
+    has set the CPU to flush subnormals converts them to zero)."""
+    u = x.view(np.uint32).astype(np.int64)
+    e = (u >> 23) & 255
+    frac = (u & 0x7FFFFF) | np.where(e > 0, 1 << 23, 0)
+    return np.where(u >> 31, -1.0, 1.0) * np.ldexp(frac.astype(np.float64),
+                                                   np.maximum(e, 1) - 150)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DENSE)
+@pytest.mark.parametrize("w_exp", [0, -118])
+def test_dense_matmul_t_tiny_values(dtype, w_exp):
+    """Values of X down to float32's subnormals, and F32 / BF16 weights below
+    2^-110 (where three bf16 pieces stop holding 24 bits), give what float32
+    products give.  Bar: cols 2^-24 of the sum of |x| |w| and cols of float32's
+    smallest subnormals, for each output."""
+    M, rows, cols = 20, 140, 96
+    rng = np.random.default_rng(3)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    if w_exp and dtype != "F16":
+        w[::3] = np.ldexp(w[::3], w_exp)
+        w[1, 5] = np.ldexp(np.float32(1.2345678), w_exp)
+    w = (w.view(np.uint32) & 0xFFFF0000).view(np.float32) if dtype == "BF16" else w
+    data = (w.astype(np.float16).view(np.uint8) if dtype == "F16" else
+            (w.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8) if dtype == "BF16"
+            else w.view(np.uint8)).reshape(-1)
+    wv = w.astype(np.float16).astype(np.float64) if dtype == "F16" else w.astype(np.float64)
+    X = synth.random_x(cols, seed=4, batch=M)
+    for i, e in enumerate((-105, -112, -116, -120, -124, -128, -140, 100, 118)):
+        X[i] = np.ldexp(X[i], e)
+    X[10, 3] = np.ldexp(np.float32(1.2345678), -115)
+    X[11] = np.ldexp(X[11], rng.integers(-125, 100, cols))
+    x64 = _f64_of_bits(X)
+    wv = wv if dtype == "F16" else _f64_of_bits(w)
+    want = x64 @ wv.T
+    bar = (np.abs(x64) @ np.abs(wv).T) * cols * 2.0 ** -24 + cols * 2.0 ** -149
+    W = DenseMatrix(data, dtype, rows, cols)
+    for prec in ("auto", "fp32"):
+        Y = _f64_of_bits(W.matmul_t(X, precision=prec))
+        bad = np.argwhere(np.abs(Y - want) > bar)
+        assert not len(bad), (prec, bad[:5], len(bad))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", DENSE)
 def test_dense_matmul_t_one_wide_row(dtype):
