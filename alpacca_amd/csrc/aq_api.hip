@@ -901,12 +901,7 @@ int matmul_t_impl(const aq_matrix *m, const float *X, int64_t M, float *Y, int p
           for (int64_t r0 = 0; r0 < M && e == hipSuccess; r0 += rows_max) {
             const float *x = static_cast<const float *>(din) + r0 * m->cols;
             const int64_t mr = std::min(rows_max, M - r0);
-            bool no_scratch = false;
-            e = aq::launch_matmul_dn(m, x, mr, yo + r0 * m->rows, m_invariant, s, &no_scratch);
-            if (no_scratch) {  // the fp32 matrix cores, which need none from about 4,096 weight rows on
-              aq::workspace_forgo();
-              e = aq::launch_matmul_t(m, x, mr, yo + r0 * m->rows, precision, s);
-            }
+            e = aq::launch_matmul_dn(m, x, mr, yo + r0 * m->rows, m_invariant, s);
           }
         } else if (small) {
           e = aq::launch_matvec_i8_batch(m, static_cast<const float *>(din), M, m->cols, yo,

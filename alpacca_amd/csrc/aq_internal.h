@@ -85,12 +85,15 @@ hipError_t launch_matmul_h(const aq_matrix *m, const float *X, int64_t M, float 
 // (aq_matmul_dn.hip), for matrices without infinities, NaNs and (F32) values
 // that three bf16 pieces do not hold (mm_dn_supported; dense_in_range looks
 // through a matrix's device copy).
-// m_invariant as for launch_matmul_h.  *no_scratch: nothing was launched, since
-// the stream's workspace cannot hold the pieces of X.
+// m_invariant as for launch_matmul_h.  Where the stream's workspace cannot hold
+// the pieces of X a slower kernel makes them as it goes, with the same bits.
 bool mm_dn_supported(const aq_matrix *m);
 hipError_t dense_in_range(const aq_matrix *m, bool *in_range);
 hipError_t launch_matmul_dn(const aq_matrix *m, const float *X, int64_t M, float *Y,
-                            bool m_invariant, hipStream_t s, bool *no_scratch);
+                            bool m_invariant, hipStream_t s);
+// The splits of K that launch_matmul_t's fp32 kernel takes for this matrix (it
+// needs scratch from two on), whatever M.
+int matmul_t_fp32_splits(const aq_matrix *m);
 // Takes back the notes of a refused workspace (a capture's, HIP's last
 // error), for a caller that goes on without one.
 void workspace_forgo();

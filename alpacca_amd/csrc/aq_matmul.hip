@@ -1022,6 +1022,16 @@ hipError_t launch_q8(const aq_matrix *m, const float *X, int64_t M, float *Y, hi
   return hipGetLastError();
 }
 
+// fp32: K stages split over up to 4 workgroups when the N tiles are few
+// (about cus / 4 per column of tiles), each split >= 8 stages; the split
+// depends on N and K only, so every output sums in the same order for any
+// M (a batched prefill gives the same results in any chunk size)
+int fp32_splits(int64_t rows, int n_stages, int cus) {
+  const int64_t ntiles = (rows + BN - 1) / BN;
+  const int splits = (int)std::min<int64_t>(4, std::max<int64_t>(1, cus / (4 * ntiles)));
+  return std::min(splits, std::max(1, n_stages / 8));
+}
+
 template <class F>
 hipError_t launch_fmt(const aq_matrix *m, const float *X, int64_t M, float *Y,
                       int precision, hipStream_t s) {
@@ -1078,15 +1088,8 @@ hipError_t launch_fmt(const aq_matrix *m, const float *X, int64_t M, float *Y,
     hipLaunchKernelGGL(k_sum_splits, dim3((unsigned)swg), dim3(256), 0, s, dst, splits, n, Y);
     return hipGetLastError();
   }
-  // fp32: K stages split over up to 4 workgroups when the N tiles are few
-  // (about cus / 4 per column of tiles), each split >= 8 stages; the split
-  // depends on N and K only, so every output sums in the same order for any
-  // M (a batched prefill gives the same results in any chunk size)
-  const int cus = device_info(m->device).cus;
   const int n_stages = (int)((m->nb_row * F::CPB * F::ELEMS + BK - 1) / BK);
-  const int64_t ntiles = (m->rows + BN - 1) / BN;
-  int splits = (int)std::min<int64_t>(4, std::max<int64_t>(1, cus / (4 * ntiles)));
-  splits = std::min(splits, std::max(1, n_stages / 8));
+  int splits = fp32_splits(m->rows, n_stages, device_info(m->device).cus);
   const int per = (n_stages + splits - 1) / splits;
   splits = (n_stages + per - 1) / per;  // no empty split
   float *dst = Y;
@@ -1106,6 +1109,11 @@ hipError_t launch_fmt(const aq_matrix *m, const float *X, int64_t M, float *Y,
 }
 
 }  // namespace
+
+int matmul_t_fp32_splits(const aq_matrix *m) {
+  return m->rows == 0 ? 1 : fp32_splits(m->rows, (int)((m->cols + BK - 1) / BK),
+                                        device_info(m->device).cus);
+}
 
 hipError_t sum_splits(const float *P, int splits, int64_t n, float *Y, hipStream_t s) {
   const int64_t swg = std::min<int64_t>((n / 4 + 255) / 256 + 1, 4096);

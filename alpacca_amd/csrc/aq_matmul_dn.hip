@@ -95,6 +95,47 @@ struct Lacking {
   int32_t k;
   float x;
 };
+// the exponent of a row from its largest finite |x|
+__device__ __forceinline__ int row_exp(float mx) {
+  return mx > 0.f ? 15 - __builtin_amdgcn_frexp_expf(mx) : 0;
+}
+// largest finite |x| and smallest |x| other than zero so far
+__device__ __forceinline__ void row_range(float x, float &mx, float &mn) {
+  mx = fmaxf(mx, __builtin_isfinite(x) ? fabsf(x) : 0.f);
+  mn = fminf(mn, x == 0.f ? INFINITY : fabsf(x));
+}
+// what the two fp16 pieces of x lack, 0 unless x is below their range
+__device__ __forceinline__ float lacking(float x, int e) {
+  const float y = __builtin_amdgcn_ldexpf(x, e);
+  if (x == 0.f || !(fabsf(y) < 0x1p-14f)) return 0.f;
+  const float hi = (float)(_Float16)y;
+  const float lo = (float)(_Float16)((y - hi) * (1 << kLoExp));
+  // (exact: the pieces hold 22 bits next to x's own)
+  return x - __builtin_amdgcn_ldexpf(fmaf(lo, 1.f / (1 << kLoExp), hi), -e);
+}
+// whether the three bf16 pieces of x cannot stand for it
+__device__ __forceinline__ bool no_pieces(float x) {
+  return !__builtin_isfinite(x) || (x != 0.f && fabsf(x) < kPieceMin);
+}
+// the pieces of four values (F16: scaled by 2^e), packed
+template <int KIND>
+__device__ __forceinline__ void cut4(float (&a)[4], uint32_t (&o)[pieces_of(KIND)][2]) {
+#pragma unroll
+  for (int p = 0; p < pieces_of(KIND); ++p)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float &x = a[2 * i], &y = a[2 * i + 1];
+      if constexpr (KIND == kF16) {
+        o[p][i] = pack_f16(x, y);
+        x = rest_of(x, (float)(_Float16)x) * (float)(1 << kLoExp);
+        y = rest_of(y, (float)(_Float16)y) * (float)(1 << kLoExp);
+      } else {
+        o[p][i] = pack_bf16(bf16_finite(x), bf16_finite(y));
+        x = rest_of(x, __uint_as_float(o[p][i] << 16));
+        y = rest_of(y, __uint_as_float(o[p][i] & 0xFFFF0000u));
+      }
+    }
+}
 template <int KIND>
 __global__ void __launch_bounds__(256)
     k_x_pieces(const float *__restrict__ X, int64_t K, int64_t Kp, uint16_t *__restrict__ xp,
@@ -115,10 +156,7 @@ __global__ void __launch_bounds__(256)
       const float4 v = *reinterpret_cast<const float4 *>(xr + j);
       const float a[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        mx = fmaxf(mx, __builtin_isfinite(a[i]) ? fabsf(a[i]) : 0.f);
-        mn = fminf(mn, a[i] == 0.f ? INFINITY : fabsf(a[i]));
-      }
+      for (int i = 0; i < 4; ++i) row_range(a[i], mx, mn);
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -132,7 +170,7 @@ __global__ void __launch_bounds__(256)
     __syncthreads();
     mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     mn = fminf(fminf(red[1][0], red[1][1]), fminf(red[1][2], red[1][3]));
-    e = mx > 0.f ? 15 - __builtin_amdgcn_frexp_expf(mx) : 0;
+    e = row_exp(mx);
     again = __builtin_amdgcn_ldexpf(mn, e) < 0x1p-14f;
   }
   for (int64_t j = 4 * (int64_t)t; j < Kp; j += 1024) {
@@ -141,13 +179,7 @@ __global__ void __launch_bounds__(256)
     float a[4] = {v.x, v.y, v.z, v.w};
     if (KIND == kF16 && again)
       for (int i = 0; i < 4; ++i) {
-        const float x = i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-        const float y = __builtin_amdgcn_ldexpf(x, e);
-        if (x == 0.f || !(fabsf(y) < 0x1p-14f)) continue;
-        const float hi = (float)(_Float16)y;
-        const float lo = (float)(_Float16)((y - hi) * (1 << kLoExp));
-        // (exact: the pieces hold 22 bits next to x's own)
-        const float d = x - __builtin_amdgcn_ldexpf(fmaf(lo, 1.f / (1 << kLoExp), hi), -e);
+        const float d = lacking(i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w, e);
         if (d == 0.f) continue;
         const int slot = atomicAdd(&n_list, 1);
         if (slot < kList) list[slot] = Lacking{(int32_t)j + i, d};
@@ -155,26 +187,13 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if constexpr (KIND == kF16) a[i] = __builtin_amdgcn_ldexpf(a[i], e);
-      else again = again || !__builtin_isfinite(a[i]) || (a[i] != 0.f && fabsf(a[i]) < kPieceMin);
+      else again = again || no_pieces(a[i]);
     }
+    uint32_t w[pieces_of(KIND)][2];
+    cut4<KIND>(a, w);
 #pragma unroll
-    for (int p = 0; p < pieces_of(KIND); ++p) {
-      uint32_t w[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        float &x = a[2 * i], &y = a[2 * i + 1];
-        if constexpr (KIND == kF16) {
-          w[i] = pack_f16(x, y);
-          x = rest_of(x, (float)(_Float16)x) * (float)(1 << kLoExp);
-          y = rest_of(y, (float)(_Float16)y) * (float)(1 << kLoExp);
-        } else {
-          w[i] = pack_bf16(bf16_finite(x), bf16_finite(y));
-          x = rest_of(x, __uint_as_float(w[i] << 16));
-          y = rest_of(y, __uint_as_float(w[i] & 0xFFFF0000u));
-        }
-      }
-      *reinterpret_cast<uint2 *>(xp + p * plane + m * Kp + j) = make_uint2(w[0], w[1]);
-    }
+    for (int p = 0; p < pieces_of(KIND); ++p)
+      *reinterpret_cast<uint2 *>(xp + p * plane + m * Kp + j) = make_uint2(w[p][0], w[p][1]);
   }
   int mark = 0;
   if constexpr (KIND != kF16) {
@@ -268,7 +287,13 @@ __device__ __forceinline__ void plain_tile(const float *X, int64_t row, const ui
   }
 }
 
-template <int KIND, int MT, int NT, int WGM, int WGN>
+// BARE: for calls that have no scratch for pieces of X.  The workgroup reads its
+// rows of X once for their exponents and marks and cuts each stage's pieces into
+// LDS itself, without a split of K: the same pieces, and bits, as otherwise
+// (14336 x 4096 at M = 512 F16 265 us, BF16 538, F32 825 against 117, 148 and
+// 332 with scratch and 650 on the fp32 kernel; at M = 2 85, 119, 152 against 42,
+// 44, 78 and 370 - 390).
+template <int KIND, int MT, int NT, int WGM, int WGN, bool BARE>
 __global__ void __launch_bounds__(64 * WGM * WGN)
     k_mm_dn(const uint8_t *W, int64_t N, int64_t K, const uint16_t *xp, int64_t plane, int64_t Kp,
             const int32_t *__restrict__ xe, const Lacking *__restrict__ xl,
@@ -302,6 +327,71 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
     const int64_t r = m0 + 8 * (i * WAVES + wave) + (lane >> 3);
     vx[i] = (uint32_t)(2 * (r < M ? r : M - 1) * Kp) + 16 * ((lane & 7) ^ (lane >> 3));
   }
+  // BARE: exponents and marks of the rows (rows past M: of row M - 1, unused)
+  int *tab = reinterpret_cast<int *>(smem + T::kLds);
+  if constexpr (BARE) {
+    for (int r = wave; r < BM; r += WAVES) {
+      const float *xr = X + (m0 + r < M ? m0 + r : M - 1) * K;
+      float mx = 0.f, mn = INFINITY;
+      bool bad = false;
+      for (int64_t j = 4 * (int64_t)lane; j < K; j += 256) {
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(xr + j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          row_range(v[i], mx, mn);
+          bad = bad || no_pieces(v[i]);
+        }
+      }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) {
+        mx = fmaxf(mx, __shfl_xor(mx, off));
+        mn = fminf(mn, __shfl_xor(mn, off));
+      }
+      int e = 0, mark = 0;
+      if constexpr (KIND == kF16) {
+        e = row_exp(mx);
+        if (__builtin_amdgcn_ldexpf(mn, e) < 0x1p-14f) {
+          for (int64_t j = lane; j < K; j += 64) mark += lacking(xr[j], e) != 0.f;
+#pragma unroll
+          for (int off = 32; off > 0; off >>= 1) mark += __shfl_xor(mark, off);
+          if (mark > kList) mark = kAgain;
+        }
+      } else if (__any(bad)) {
+        mark = kAgain;
+      }
+      if (lane == 0) tab[r] = 16 * e + mark;
+    }
+    __syncthreads();
+  }
+  // BARE: the pieces of X of a stage, laid out as the DMAs lay them out
+  auto cut_stage = [&](int st, int buf) {
+    for (int q = tid; q < BM * 8; q += T::kThreads) {
+      const int r = q >> 3, c = q & 7;
+      const int64_t col = (int64_t)st * 64 + 8 * c;
+      float a[2][4] = {};
+      if (col < K) {
+        const float *p = X + (m0 + r < M ? m0 + r : M - 1) * K + col;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) a[h][i] = p[4 * h + i];
+      }
+      if constexpr (KIND == kF16) {
+        const int e = tab[r] >> 4;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) a[h][i] = __builtin_amdgcn_ldexpf(a[h][i], e);
+      }
+      uint32_t w0[NX][2], w1[NX][2];
+      cut4<KIND>(a[0], w0);
+      cut4<KIND>(a[1], w1);
+#pragma unroll
+      for (int p = 0; p < NX; ++p)
+        *reinterpret_cast<u32x4 *>(smem + buf * T::kX + p * BM * 128 + r * 128 + 16 * (c ^ (r & 7))) =
+            u32x4{w0[p][0], w0[p][1], w1[p][0], w1[p][1]};
+    }
+  };
   // W stage: BN rows of kRow bytes, chunk c of row r in slot c ^ (r & 7); rows
   // past N repeat row N - 1.  Where K ends inside a stage (K is a multiple of
   // 32), the chunks past it repeat the stage's first half: x is zero there.
@@ -320,8 +410,9 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
   }
   static_assert(RPD * WAVES % 8 == 0, "one swizzle per lane");
   auto dma_stage = [&](int st, int buf) {
+    if constexpr (BARE) cut_stage(st, buf);
 #pragma unroll
-    for (int i = 0; i < XI; ++i)
+    for (int i = 0; i < (BARE ? 0 : XI); ++i)
       dma16(lds0 + buf * T::kX + 1024 * (i * WAVES + wave), vx[i % XR],
             reinterpret_cast<const uint8_t *>(xp) + 2 * plane * ((i * WAVES) / XP) + 128 * (int64_t)st);
     const uint32_t back = (int64_t)st * 64 + 64 > K ? tail : 0;
@@ -383,11 +474,12 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
   // behind a stage's barrier (in the stores their latency would be 0.3 us of every
   // call)
   const int64_t my_row = m0 + wm * MT * 16 + lane;
-  int mark = lane < MT * 16 && my_row < M ? xe[my_row] : 0;
+  int mark = 0;
+  if (lane < MT * 16 && my_row < M) mark = BARE ? tab[wm * MT * 16 + lane] : xe[my_row];
   dma_stage(s_begin, 0);
   if (s_begin + 1 < s_end) {
     dma_stage(s_begin + 1, 1);
-    dma_barrier<XI + WI>();
+    dma_barrier<(BARE ? 0 : XI) + WI>();
   } else {
     dma_barrier<0>();
   }
@@ -464,15 +556,26 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
         for (int rr = 0; rr < 4; ++rr) {
           const int64_t row = row0 + 4 * g + rr;
           const int count = todo[rr] == kAgain ? 0 : todo[rr];
-#pragma unroll 1
-          for (int c = 0; c < count; ++c) {
-            const Lacking l = xl[row * kList + c];
-            if (l.k < k_begin || l.k >= k_end) continue;  // another split's
+          auto add = [&](int64_t k, float x) {
             for (int j = 0; j < NT; ++j) {
               const int64_t n = n0 + (wn * NT + j) * 16 + c16;
               if (n < N)
-                Y[row * N + n] = fmaf(l.x, (float)reinterpret_cast<const _Float16 *>(W)[n * K + l.k],
+                Y[row * N + n] = fmaf(x, (float)reinterpret_cast<const _Float16 *>(W)[n * K + k],
                                       Y[row * N + n]);
+            }
+          };
+          if constexpr (BARE) {
+            const int e = __shfl(mark, i * 16 + 4 * g + rr) >> 4;
+#pragma unroll 1
+            for (int64_t k = 0; count > 0 && k < K; ++k) {
+              const float d = lacking(X[row * K + k], e);
+              if (d != 0.f) add(k, d);
+            }
+          } else {
+#pragma unroll 1
+            for (int c = 0; c < count; ++c) {
+              const Lacking l = xl[row * kList + c];
+              if (l.k >= k_begin && l.k < k_end) add(l.k, l.x);  // (else another split's)
             }
           }
         }
@@ -505,19 +608,28 @@ struct DnLaunch {
   int splits, per;
   hipStream_t s;
 };
-template <int KIND, int MT, int NT, int WGM, int WGN>
+template <int KIND, int MT, int NT, int WGM, int WGN, bool BARE = false>
 hipError_t launch_tile(const DnLaunch &a) {
   using T = DnTile<KIND, MT, NT, WGM, WGN>;
   const int mt = (int)((a.M + T::BM - 1) / T::BM), nt = (int)((a.m->rows + T::BN - 1) / T::BN);
   const dim3 grid((unsigned)(((int64_t)mt * nt + 7) / 8 * 8), 1, (unsigned)a.splits);
-  auto kern = k_mm_dn<KIND, MT, NT, WGM, WGN>;
-  if (hipError_t e = set_dynamic_lds(reinterpret_cast<const void *>(kern), T::kLds)) return e;
-  hipLaunchKernelGGL(kern, grid, dim3(T::kThreads), T::kLds, a.s, a.m->planes.p[0], a.m->rows,
+  constexpr int lds = T::kLds + (BARE ? T::BM * 4 : 0);
+  auto kern = k_mm_dn<KIND, MT, NT, WGM, WGN, BARE>;
+  if (hipError_t e = set_dynamic_lds(reinterpret_cast<const void *>(kern), lds)) return e;
+  hipLaunchKernelGGL(kern, grid, dim3(T::kThreads), lds, a.s, a.m->planes.p[0], a.m->rows,
                      a.m->cols, a.xp, a.plane, a.Kp, a.xe, a.xl, a.X, a.M, a.dst, a.per, mt, nt);
   return hipGetLastError();
 }
 template <int KIND>
 hipError_t launch_shape(int shape, const DnLaunch &a) {
+  if (!a.xp) {
+    // without scratch: 14336 x 4096, 32 against 64 rows a tile, M = 64 F16 104
+    // against 111 us, F32 175 / 207, M = 512 322 / 265, 1173 / 825 (BF16 538 / 621)
+    if constexpr (KIND != kBF16) {
+      if (a.M > 128) return launch_tile<KIND, 2, 2, 2, 4, true>(a);
+    }
+    return launch_tile<KIND, 2, 2, 1, 4, true>(a);
+  }
   switch (shape) {
     case 0:
       if constexpr (KIND != kF32) return launch_tile<KIND, 4, 4, 2, 4>(a);
@@ -586,47 +698,59 @@ bool mm_dn_supported(const aq_matrix *m) {
 }
 
 hipError_t launch_matmul_dn(const aq_matrix *m, const float *X, int64_t M, float *Y,
-                            bool m_invariant, hipStream_t s, bool *no_scratch) {
-  *no_scratch = false;
+                            bool m_invariant, hipStream_t s) {
   if (M == 0 || m->rows == 0) return hipSuccess;
   const int kind = m->dtype == AQ_F16 ? kF16 : m->dtype == AQ_BF16 ? kBF16 : kF32;
   const int64_t K = m->cols, N = m->rows, Kp = (K + 63) / 64 * 64;
   if (!mm_dn_supported(m) || (double)M * Kp * 2 >= 2147483648.0) return hipErrorInvalidValue;
   const int units = (int)(Kp / 64), cus = device_info(m->device).cus;
-  int shape = 0, splits = 1;
-  choose_tile(kModel, kind, M, N, units, 1, 4, cus, m_invariant ? 1 : 16, shape, splits);
-  // AQ_MATMUL_TILE (tests): the shape itself, where the kind has it
-  if (const char *env = getenv("AQ_MATMUL_TILE")) {
-    const int v = atoi(env);
-    if (v >= 0 && v < kTileShapes && kTiles[v].one[kind] > 0.f) shape = v;
-  }
-  const int per = (units + splits - 1) / splits;
-  splits = (units + per - 1) / per;
   auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
   const int64_t plane = M * Kp;
   const size_t xb = al((size_t)pieces_of(kind) * plane * 2), eb = al((size_t)M * 4),
                lb = kind == kF16 ? al((size_t)M * kList * sizeof(Lacking)) : 0;
-  const size_t part = splits > 1 ? (size_t)splits * M * N * 4 : 0;
-  uint8_t *ws = static_cast<uint8_t *>(workspace(m->device, s, xb + eb + lb + part));
-  if (!ws) {
-    *no_scratch = true;
-    return hipErrorOutOfMemory;
+  DnLaunch a{m, nullptr, plane, Kp, nullptr, nullptr, X, M, Y, 1, units, s};
+  int shape = 0;
+  uint8_t *ws = nullptr;
+  // with a split of K, without one (whose partials the scratch may not hold)
+  for (int most = m_invariant ? 1 : 16;; most = 1) {
+    int splits = 1;
+    choose_tile(kModel, kind, M, N, units, 1, 4, cus, most, shape, splits);
+    // AQ_MATMUL_TILE (tests): the shape itself, where the kind has it
+    if (const char *env = getenv("AQ_MATMUL_TILE")) {
+      const int v = atoi(env);
+      if (v >= 0 && v < kTileShapes && kTiles[v].one[kind] > 0.f) shape = v;
+    }
+    a.per = (units + splits - 1) / splits;
+    a.splits = (units + a.per - 1) / a.per;
+    const size_t part = a.splits > 1 ? (size_t)a.splits * M * N * 4 : 0;
+    ws = static_cast<uint8_t *>(workspace(m->device, s, xb + eb + lb + part));
+    if (ws || most == 1) break;
+    workspace_forgo();
   }
-  uint16_t *xp = reinterpret_cast<uint16_t *>(ws);
-  int32_t *xe = reinterpret_cast<int32_t *>(ws + xb);
-  Lacking *xl = reinterpret_cast<Lacking *>(ws + xb + eb);
-  float *dst = splits > 1 ? reinterpret_cast<float *>(ws + xb + eb + lb) : Y;
+  if (ws) {
+    uint16_t *xp = reinterpret_cast<uint16_t *>(ws);
+    int32_t *xe = reinterpret_cast<int32_t *>(ws + xb);
+    Lacking *xl = reinterpret_cast<Lacking *>(ws + xb + eb);
+    if (a.splits > 1) a.dst = reinterpret_cast<float *>(ws + xb + eb + lb);
+    a.xp = xp;
+    a.xe = xe;
+    a.xl = xl;
 #define AQ_XP(k) \
   hipLaunchKernelGGL(k_x_pieces<k>, dim3((unsigned)M), dim3(256), 0, s, X, K, Kp, xp, plane, xe, xl)
-  if (kind == kF16) AQ_XP(kF16);
-  else AQ_XP(kBF16);  // (the same pieces for F32)
+    if (kind == kF16) AQ_XP(kF16);
+    else AQ_XP(kBF16);  // (the same pieces for F32)
 #undef AQ_XP
-  const DnLaunch a{m, xp, plane, Kp, xe, xl, X, M, dst, splits, per, s};
+  } else {
+    // Few weight rows have always needed scratch (the fp32 kernel splits K for
+    // them): refused without, as before.
+    if (matmul_t_fp32_splits(m) > 1) return hipErrorOutOfMemory;
+    workspace_forgo();
+  }
   const hipError_t e = kind == kF16    ? launch_shape<kF16>(shape, a)
                        : kind == kBF16 ? launch_shape<kBF16>(shape, a)
                                        : launch_shape<kF32>(shape, a);
-  if (e != hipSuccess || splits == 1) return e;
-  return sum_splits(dst, splits, M * N, Y, s);
+  if (e != hipSuccess || a.splits == 1) return e;
+  return sum_splits(a.dst, a.splits, M * N, Y, s);
 }
 
 }  // namespace aq

@@ -197,9 +197,9 @@ int aq_matvec_fused(const aq_matrix *const *ms, int n, const float *x,
  * rows of X sharing one weight stream (the accuracy of aq_matvec; other
  * matrices up to 32 rows, 63 for 2^24 weights or more); dense matrices of
  * finite values (F32: none below 2^-110 but zeros) on 16-bit MFMA in exact
- * pieces (one row: the fp32 matvec);
- * the rest on fp32 MFMA.  AQ_PREC_FP32 gives every M the same bits (the
- * batched prefill step's precision); AQ_PREC_BF16 is an opt-in. */
+ * pieces (one row: the fp32 matvec); the rest on fp32 MFMA.  AQ_PREC_FP32 gives every M the same bits (the
+ * batched prefill step's precision), with and without scratch on the stream;
+ * AQ_PREC_BF16 is an opt-in. */
 int aq_matmul_t(const aq_matrix *m, const float *X, int64_t M, float *Y,
                 int precision, int flags, void *stream);
 

@@ -87,10 +87,10 @@ def test_capture_refuses_scratch_growth():
 
 @pytest.mark.parametrize("dtype", ["F16", "BF16", "F32"])
 def test_dense_capture_without_scratch(dtype):
-    """A dense matmul_t captured on a stream that holds no scratch runs on the
-    fp32 matrix cores, which need none for this many weight rows; the error
-    of a call that does need some is not left behind.  Bar 1e-5 of max|Y|
-    between the two kernels' fp32 sums over 256 columns."""
+    """A dense matmul_t captured on a stream that holds no scratch runs without
+    any for this many weight rows; the error of a call that does need some is
+    not left behind.  Bar 1e-5 of max|Y| between the fp32 sums over 256 columns
+    in two orders."""
     d = torch.device("cuda", 0)
     rows, cols, M = 4224, 256, 5
     W = DenseMatrix(synth.dense_values_bytes(dtype, rows, cols, seed=4), dtype, rows, cols)
@@ -112,6 +112,47 @@ def test_dense_capture_without_scratch(dtype):
         assert np.abs(Y.cpu().numpy() - want).max() < 1e-5 * np.abs(want).max()
     with pytest.raises(ValueError):  # its own message, not the refused scratch
         W.matmul_t_device(X.data_ptr(), -1, Y.data_ptr(), h)
+
+
+@pytest.mark.parametrize("M", [5, 70])
+@pytest.mark.parametrize("dtype", ["F16", "BF16", "F32"])
+def test_dense_fp32_same_bits_without_scratch(dtype, M):
+    """A dense matmul_t at fp32 gives the same bits whether the stream holds
+    scratch for it or not, and for any M: captured without any, and in an
+    eager call; rows that are corrected or formed again among them (the
+    largest and smallest floats, an infinity, a NaN, a wide range)."""
+    d = torch.device("cuda", 0)
+    rows, cols = 4200, 352
+    W = DenseMatrix(synth.dense_values_bytes(dtype, rows, cols, seed=7), dtype, rows, cols)
+    Xh = synth.random_x(cols, seed=8, batch=M)
+    Xh[0, 9] = 1e9
+    Xh[1, 3], Xh[1, 300:303] = 1e5, 1e-6
+    Xh[2, 5] = np.inf
+    Xh[3, 6], Xh[3, 7] = 3.4e38, 1e-36
+    if M > 20:
+        Xh[20, 8] = np.nan
+        Xh[33] = 0.0
+        Xh[64] *= np.float32(1e-36)
+    X = torch.from_numpy(Xh).to(d)
+    Y = torch.empty((M, rows), device=d)
+    s = torch.cuda.Stream(d)
+    h = s.cuda_stream
+    _lib.check(_lib.ensure_device().aq_release_workspace(ctypes.c_void_p(h)))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        W.matmul_t_device(X.data_ptr(), M, Y.data_ptr(), h, "fp32")
+    got = []
+    for _ in range(3):
+        Y.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            g.replay()
+        s.synchronize()
+        got.append(Y.cpu().numpy().view(np.uint32))
+    want = W.matmul_t(Xh, precision="fp32").view(np.uint32)
+    assert all(np.array_equal(y, want) for y in got)
+    cut = np.concatenate([W.matmul_t(Xh[a:b], precision="fp32") for a, b in ((0, 3), (3, M))])
+    assert np.array_equal(cut.view(np.uint32), want)
 
 
 @pytest.mark.parametrize("dtype", ["F16", "F32", "Q4_K"])
