@@ -896,8 +896,11 @@ int matmul_t_impl(const aq_matrix *m, const float *X, int64_t M, float *Y, int p
           return hipSuccess;
         } else if (dense1) {
           e = aq::launch_matvec(m, static_cast<const float *>(din), yo, s);
-        } else if (dense16) {  // in slices of rows for the same reason
-          const int64_t rows_max = std::max<int64_t>(1, ((int64_t)1 << 29) / (m->cols + 32));
+        } else if (dense16) {
+          // in slices of rows whose pieces (at most three, and 68 bytes) stay below 2^28:
+          // what the stream's scratch keeps; whole tiles where there are several
+          int64_t rows_max = std::max<int64_t>(1, ((int64_t)1 << 28) / (6 * (m->cols + 32) + 80));
+          if (rows_max > 256) rows_max = rows_max / 256 * 256;
           for (int64_t r0 = 0; r0 < M && e == hipSuccess; r0 += rows_max) {
             const float *x = static_cast<const float *>(din) + r0 * m->cols;
             const int64_t mr = std::min(rows_max, M - r0);

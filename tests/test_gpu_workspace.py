@@ -155,6 +155,31 @@ def test_dense_fp32_same_bits_without_scratch(dtype, M):
     assert np.array_equal(cut.view(np.uint32), want)
 
 
+def test_dense_scratch_is_bounded():
+    """A dense matmul_t of many rows of X runs in slices: the stream's scratch for
+    their pieces stays at 256 MiB (the pieces of all 24,000 rows: 590 MB), and a
+    slice's end changes no bits at fp32."""
+    d = torch.device("cuda", 0)
+    rows, cols, M = 96, 4096, 24000
+    W = DenseMatrix(synth.dense_values_bytes("F32", rows, cols, seed=9), "F32", rows, cols)
+    X = torch.randn((M, cols), device=d)
+    Y = torch.empty((M, rows), device=d)
+    s = torch.cuda.Stream(d)
+    h = s.cuda_stream
+    W.matmul_t_device(X.data_ptr(), 2, Y.data_ptr(), None, "fp32")
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info(d)[0]
+    W.matmul_t_device(X.data_ptr(), M, Y.data_ptr(), h, "fp32")
+    s.synchronize()
+    assert free - torch.cuda.mem_get_info(d)[0] <= (256 + 64) << 20
+    got = Y.cpu().numpy()
+    per = (1 << 28) // (6 * (cols + 32) + 80) // 256 * 256
+    for r in (0, per - 3, 2 * per - 3, M - 6):
+        want = W.matmul_t(X[r:r + 6].cpu().numpy(), precision="fp32")
+        assert np.array_equal(got[r:r + 6].view(np.uint32), want.view(np.uint32)), r
+    _lib.check(_lib.ensure_device().aq_release_workspace(ctypes.c_void_p(h)))
+
+
 @pytest.mark.parametrize("dtype", ["F16", "F32", "Q4_K"])
 def test_threads_share_a_stream(dtype):
     """Host threads that call on one stream (calls on host arrays all run on
