@@ -873,8 +873,9 @@ __global__ void __launch_bounds__(256)
 // accumulator (what is dropped is below 2^-25 of it), so products and sums
 // keep fp32's accuracy at 6/16 of the fp32 matrix cores' time
 // (v_mfma_f32_16x16x32_bf16 against 16x16x4f32).  No scaling is needed: bf16
-// has fp32's exponent range.  Rows that meet an infinity or a NaN are formed
-// again in fp32 at the end.
+// has fp32's exponent range.  Rows that meet an infinity or a NaN, or values
+// whose 24 bits the pieces do not hold where that shows, are formed again in fp32
+// at the end.
 //
 // Grid: one workgroup of NW waves per (16 NW (token, head) rows, kv head); a
 // wave owns 16 rows (16 / G tokens times the G heads) and keeps the online
@@ -924,7 +925,7 @@ __device__ __forceinline__ void pieces3_cut(float a, float b, uint32_t (&o)[3]) 
   }
 }
 template <int HD, int G, int NW>
-__global__ void __launch_bounds__(64 * NW)
+__global__ void __launch_bounds__(64 * NW, HD == 64 ? 3 : 1)
     k_attn_prefill_mfma(const float *__restrict__ q, const float *__restrict__ kc,
                         const float *__restrict__ vc, const aq_decode_state *st, int64_t pos0,
                         int64_t n_ctx, int64_t T, float scale, int tiles, int fold,
@@ -955,6 +956,7 @@ __global__ void __launch_bounds__(64 * NW)
   const int64_t t_row = tw + r16 / G;
   const int h_row = kvh * G + r16 % G;
   bf16x8_ qf[KS][3];
+  uint32_t q_low = ~0u, q_high = 0;
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     f4v_ v[2] = {f4v_{0.f, 0.f, 0.f, 0.f}, f4v_{0.f, 0.f, 0.f, 0.f}};
@@ -964,6 +966,12 @@ __global__ void __launch_bounds__(64 * NW)
       v[0] = qr[0];
       v[1] = qr[1];
     }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {  // (bits without the sign, times 2, less 1: zero comes last)
+      const uint32_t u = (__float_as_uint(v[i >> 2][i & 3]) << 1) - 1;
+      q_low = min(q_low, u);
+      q_high = max(q_high, u + 1);
+    }
     uint32_t w[4][3];
 #pragma unroll
     for (int i = 0; i < 4; ++i) pieces3(v[i >> 1][2 * (i & 1)], v[i >> 1][2 * (i & 1) + 1], w[i]);
@@ -971,6 +979,11 @@ __global__ void __launch_bounds__(64 * NW)
     for (int p = 0; p < 3; ++p)
       qf[ks][p] = __builtin_bit_cast(bf16x8_, u32x4_{w[0][p], w[1][p], w[2][p], w[3][p]});
   }
+  // a value of the row's q outside 2^-110 .. 2^100, not zero (here: the compiler
+  // would sink the comparisons to the use, with q in 32 registers until then)
+  asm volatile("" : "+v"(q_low), "+v"(q_high));
+  const bool q_far = q_low < (__builtin_bit_cast(uint32_t, 0x1p-110f) << 1) - 1 ||
+                     q_high > (__builtin_bit_cast(uint32_t, 0x1p100f) << 1);
   int64_t t_last = (int64_t)tile * TPB + TPB - 1;
   t_last = t_last < T ? t_last : T - 1;
   int64_t p_last = pb + t_last;  // the last position any row of the block sees
@@ -1111,15 +1124,26 @@ __global__ void __launch_bounds__(64 * NW)
   // lane (r16, cg) of tile ht holds O^T[16 ht + 4 cg + r][row r16]
   float den = add_xor<16>(l);
   den = add_xor<32>(den);
-  // Rows whose pieces were not finite (an infinity leaves inf - inf, a value
-  // within 2^-9 of the largest rounds up to one, and what is masked for the row
-  // counts too) come out NaN and are formed again in fp32 over what they see.
+  // Rows that the pieces do not serve are formed again in fp32 over what they see:
+  //   NaN: pieces that are not finite (an infinity leaves inf - inf, a value
+  //     within 2^-9 of the largest rounds up to one, and what is masked for the
+  //     row counts too);
+  //   pieces end at bf16's last subnormal bit, 2^-133, so an operand is off by up
+  //     to 2^-134: in the scores that matters only against a q or K above 2^100,
+  //     which takes a q above it or a q below 2^-110 (q_far); in the output only
+  //     where that is below 2^-110 itself (V below 2^-134 counts as zero there).
   float chk = den - den;
+  uint32_t low = ~0u;  // the smallest |o| other than zero (as bits, times 2, less 1)
 #pragma unroll
   for (int ht = 0; ht < NHT; ++ht)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) chk = fmaf(o[ht][r], 0.f, chk);
-  const bool again = t_row < T && add_xor<32>(add_xor<16>(chk)) != 0.f;
+    for (int r = 0; r < 4; ++r) {
+      chk = fmaf(o[ht][r], 0.f, chk);
+      low = min(low, (__float_as_uint(o[ht][r]) << 1) - 1);
+    }
+  if (q_far || low < (__float_as_uint(0x1p-110f * den) << 1) - 1) chk = 1.f;
+  chk = add_xor<32>(add_xor<16>(chk));
+  const bool again = t_row < T && chk != 0.f;
   if (__any(again)) {
 #pragma clang fp contract(off)  // (d - mn of the maximum itself is 0, not d's rounding)
     int64_t last = -1;          // the row's last position

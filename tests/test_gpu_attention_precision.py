@@ -140,3 +140,53 @@ def test_attention_batch_nonfinite(hd, T):
                 assert np.array_equal(want[~fin], g[~fin], equal_nan=True), (t, h)
                 bar = np.abs(V[kv, :n].astype(np.float64)).max(axis=0)
                 assert (np.abs(g - want)[fin] <= 1e-5 * bar[fin]).all(), (t, h)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("what", ["v", "v_late", "k", "q", "q_some"])
+def test_attention_batch_tiny_values(hd, what):
+    """Values whose 24 bits three bf16 pieces do not hold (below 2^-110): V of
+    that size (v_late: in one dimension, from position 70 on), and K or q of that
+    size against q or K so large that their scores matter (q_some: in every fifth
+    row, one dimension).  Bar 1e-5 max|V| of each dimension against float64, as
+    above, and the same bits when the tokens come in several calls."""
+    n_head, n_kv, T = 8, 2, 100
+    rng = np.random.default_rng(hd)
+    q = rng.standard_normal((T, n_head, hd)).astype(np.float32)
+    K = rng.standard_normal((n_kv, T, hd)).astype(np.float32)
+    V = rng.standard_normal((n_kv, T, hd)).astype(np.float32)
+    if what == "v":
+        V = np.ldexp(V, -118)
+    elif what == "v_late":
+        V[:, :70, 3] = 0.0
+        V[:, 70:, 3] = np.ldexp(V[:, 70:, 3], -118)
+    elif what == "q_some":
+        q[::5, :, 1] = np.ldexp(q[::5, :, 1], -118)
+        q[1::5, :, 1] = q[2::5, :, 1] = q[3::5, :, 1] = q[4::5, :, 1] = 0.0
+        K[:, ::2, 1] = np.ldexp(np.abs(K[:, ::2, 1]), 119)
+    else:
+        q = np.ldexp(q, -116 if what == "q" else 115)
+        K = np.ldexp(K, 118 if what == "q" else -117)
+    qd, kc, vc = (torch.from_numpy(a).to("cuda") for a in (q, K, V))
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    lib = _lib.ensure_device()
+
+    def run(cuts):
+        out = torch.empty((T, n_head, hd), device="cuda")
+        for a, b in zip(cuts, cuts[1:]):
+            _lib.check(lib.aq_attention_batch(p(qd[a:b]), p(kc), p(vc), b - a, n_head, n_kv, hd,
+                                              T, None, a, p(out[a:b]), None))
+        return out.cpu().numpy()
+
+    got = run([0, T])
+    assert np.array_equal(got.view(np.uint32), run([0, 3, 37, 72, T]).view(np.uint32))
+    for t in range(T):
+        for h in range(n_head):
+            kv = h // (n_head // n_kv)
+            s = (K[kv, :t + 1].astype(np.float64) @ q[t, h].astype(np.float64)) / math.sqrt(hd)
+            w = np.exp(s - s.max())
+            v = V[kv, :t + 1].astype(np.float64)
+            want = (w / w.sum()) @ v
+            bar = 1e-5 * np.abs(v).max(axis=0)
+            err = np.abs(got[t, h].astype(np.float64) - want)
+            assert (err <= bar).all(), (t, h, (err - bar).max())
