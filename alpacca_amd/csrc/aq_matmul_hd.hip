@@ -212,8 +212,11 @@ struct HdB32 {
 // ---- tile kernel -----------------------------------------------------------------
 constexpr int NP = 2;  // pieces of X
 
+// XB: X stages in LDS.  A group is four stages and stage c of any group uses
+// buffer c % XB, so XB divides four.
 template <class F, int MT, int NT, int WGM, int WGN, int XB>
 struct HdTile {
+  static_assert(XB == 2 || XB == 4, "whole turns of the X buffers per group");
   static constexpr int kWaves = WGM * WGN, kThreads = 64 * kWaves;
   static constexpr int BM = WGM * MT * 16, BN = WGN * NT * 16;
   static constexpr int kParts = F::kF0 + F::kF1 + F::kF2 + F::kPad;  // 16-byte chunks of a row
@@ -578,7 +581,20 @@ hipError_t launch_shape(int shape, const HdLaunch &a) {
     case 1: return launch_tile<F, 4, 2, 2, 4, 2>(a);
     case 2: return launch_tile<F, 2, 2, 2, 4, 2>(a);
     case 3: return launch_tile<F, 2, 2, 1, 4, 2>(a);
-    default: return launch_tile<F, 1, 2, 1, 4, 2>(a);
+    default: {
+      // A stage of 16 rows is shorter than an X stage's way into LDS, so three are
+      // under way at a time where the LDS for it costs no second workgroup on a
+      // CU: always but for Q8_0, there where the launch has none (4096 x 14336
+      // unsplit, M = 16: Q8_0 90.2 us with one, 77.3 with three, Q4_K 90.8 / 75.8;
+      // split, two Q8_0 workgroups to a CU: 23.8 / 27.2).
+      using T4 = HdTile<F, 1, 2, 1, 4, 4>;
+      constexpr bool pair = 2 * T4::kLds <= 160 * 1024;
+      if constexpr (!pair) {
+        const int64_t wgs = (a.M + T4::BM - 1) / T4::BM * ((a.m->rows + T4::BN - 1) / T4::BN) * a.splits;
+        if (wgs > device_info(a.m->device).cus) return launch_tile<F, 1, 2, 1, 4, 2>(a);
+      }
+      return launch_tile<F, 1, 2, 1, 4, 4>(a);
+    }
   }
 }
 

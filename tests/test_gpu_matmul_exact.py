@@ -488,3 +488,19 @@ def test_tile_kernel_layouts_agree(dtype, layout):
     want, norms = _f64(data, rows, cols, X, dtype)
     Y = QuantMatrix(data, dtype, rows, cols, layout=layout).matmul_t(X)
     assert normalized_error(Y, want, norms, X) < TILE_TOL
+
+
+@pytest.mark.parametrize("dtype", ["Q8_0", "Q4_K"])
+@pytest.mark.parametrize("rows,cols", [(2000, 1280), (33000, 256), (33000, 768)])
+def test_tile_16_rows_stages_ahead(dtype, rows, cols, monkeypatch):
+    """The 16-row tile with three X stages under way, and for Q8_0 with more
+    workgroups than CUs with one, over one to five groups of columns: the bits
+    of the 32-row tile."""
+    M = 9
+    qm = QuantMatrix(synth.random_matrix_bytes(dtype, rows, cols, seed=3), dtype, rows, cols)
+    X = synth.random_x(cols, seed=4, batch=M)
+    got = []
+    for shape in (3, 4):
+        monkeypatch.setenv("AQ_MATMUL_TILE", str(shape))
+        got.append(qm.matmul_t(X, precision="fp32").view(np.uint32))
+    assert np.array_equal(got[0], got[1])
