@@ -25,6 +25,7 @@ library, and a missing library or GPU raises instead of falling back.
 from __future__ import annotations
 
 import ctypes
+import gc
 import math
 from dataclasses import dataclass
 
@@ -654,15 +655,22 @@ class Model:
         """A HIP graph of fn on self.stream, for launches that the stream has
         run before (their workspace is there).  Work queued on the stream
         runs on meanwhile: unlike torch.cuda.graph, nothing here waits for
-        the device."""
+        the device, or collects garbage first - so none is collected during
+        the capture either, where freeing a matrix or a graph is an error."""
         torch = self.torch
+        collecting = gc.isenabled()
         g = torch.cuda.CUDAGraph()
         with torch.cuda.stream(self.stream):
-            g.capture_begin()
+            gc.disable()
             try:
-                fn()
+                g.capture_begin()
+                try:
+                    fn()
+                finally:
+                    g.capture_end()
             finally:
-                g.capture_end()
+                if collecting:
+                    gc.enable()
         return g
 
 
