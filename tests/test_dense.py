@@ -218,6 +218,38 @@ def test_dense_matmul_t_nonfinite(dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bad_w", [False, True])
+@pytest.mark.parametrize("dtype", DENSE)
+def test_dense_matmul_t_nonfinite_split(dtype, bad_w):
+    """Infinities and NaNs with K split over workgroups (few weight rows, 4096
+    columns): of the tile kernel, where every split forms its own columns of a
+    row again, and, with an infinite weight, of the fp32 kernel.  Bar as above."""
+    M, rows, cols = 6, 40, 4096
+    rng = np.random.default_rng(5)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    w = (w.view(np.uint32) & 0xFFFF0000).view(np.float32)
+    if bad_w:
+        w[7, 3000] = np.inf
+    data = (w.astype(np.float16).view(np.uint8) if dtype == "F16" else
+            (w.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8) if dtype == "BF16"
+            else w.view(np.uint8)).reshape(-1)
+    wv = w.astype(np.float16).astype(np.float64) if dtype == "F16" else w.astype(np.float64)
+    X = synth.random_x(cols, seed=6, batch=M)
+    X[1, 70], X[2, 4000] = np.inf, np.nan
+    X[3, 100], X[3, 3900] = np.inf, -np.inf
+    X[4, 5], X[4, 2500] = np.inf, 1e-36
+    with np.errstate(invalid="ignore"):
+        want = X.astype(np.float64) @ wv.T
+        bar = (np.abs(X).astype(np.float64) @ np.abs(wv).T) * cols * 2.0 ** -24
+    W = DenseMatrix(data, dtype, rows, cols)
+    for prec in ("auto", "fp32"):
+        Y = W.matmul_t(X, precision=prec).astype(np.float64)
+        fin = np.isfinite(want)
+        assert np.array_equal(want[~fin], Y[~fin], equal_nan=True), prec
+        assert (np.abs(Y[fin] - want[fin]) <= bar[fin]).all(), prec
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", DENSE)
 @pytest.mark.parametrize("cols", [64, 2080])
 def test_dense_matmul_t_wide_range_rows(dtype, cols, monkeypatch):
