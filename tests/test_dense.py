@@ -17,6 +17,7 @@ from alpacca_amd import gguf, synth
 from alpacca_amd.qmatrix import DENSE_DTYPES, DenseMatrix, QuantMatrix
 from oracle.qmatrix_ref import DenseRef, normalized_error
 from oracle.quants_ref import dense_decode
+from tests.f64 import f64_of_bits
 
 DENSE = ("F32", "F16", "BF16")
 
@@ -301,16 +302,6 @@ def test_dense_matmul_t_wide_range_rows(dtype, cols, monkeypatch):
                 assert np.array_equal(Y.view(np.uint32), first.view(np.uint32)), shape
 
 
-def _f64_of_bits(x):
-    """float32 values as float64 from their bits (a process in which some library
-    has set the CPU to flush subnormals converts them to zero)."""
-    u = x.view(np.uint32).astype(np.int64)
-    e = (u >> 23) & 255
-    frac = (u & 0x7FFFFF) | np.where(e > 0, 1 << 23, 0)
-    return np.where(u >> 31, -1.0, 1.0) * np.ldexp(frac.astype(np.float64),
-                                                   np.maximum(e, 1) - 150)
-
-
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", DENSE)
 @pytest.mark.parametrize("w_exp", [0, -118])
@@ -335,13 +326,13 @@ def test_dense_matmul_t_tiny_values(dtype, w_exp):
         X[i] = np.ldexp(X[i], e)
     X[10, 3] = np.ldexp(np.float32(1.2345678), -115)
     X[11] = np.ldexp(X[11], rng.integers(-125, 100, cols))
-    x64 = _f64_of_bits(X)
-    wv = wv if dtype == "F16" else _f64_of_bits(w)
+    x64 = f64_of_bits(X)
+    wv = wv if dtype == "F16" else f64_of_bits(w)
     want = x64 @ wv.T
     bar = (np.abs(x64) @ np.abs(wv).T) * cols * 2.0 ** -24 + cols * 2.0 ** -149
     W = DenseMatrix(data, dtype, rows, cols)
     for prec in ("auto", "fp32"):
-        Y = _f64_of_bits(W.matmul_t(X, precision=prec))
+        Y = f64_of_bits(W.matmul_t(X, precision=prec))
         bad = np.argwhere(np.abs(Y - want) > bar)
         assert not len(bad), (prec, bad[:5], len(bad))
 

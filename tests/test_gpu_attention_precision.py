@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 
 from alpacca_amd import _lib
+from tests.f64 import f64_of_bits
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -180,13 +181,14 @@ def test_attention_batch_tiny_values(hd, what):
 
     got = run([0, T])
     assert np.array_equal(got.view(np.uint32), run([0, 3, 37, 72, T]).view(np.uint32))
+    got, q, K, V = (f64_of_bits(a) for a in (got, q, K, V))
     for t in range(T):
         for h in range(n_head):
             kv = h // (n_head // n_kv)
-            s = (K[kv, :t + 1].astype(np.float64) @ q[t, h].astype(np.float64)) / math.sqrt(hd)
+            s = (K[kv, :t + 1] @ q[t, h]) / math.sqrt(hd)
             w = np.exp(s - s.max())
-            v = V[kv, :t + 1].astype(np.float64)
+            v = V[kv, :t + 1]
             want = (w / w.sum()) @ v
             bar = 1e-5 * np.abs(v).max(axis=0)
-            err = np.abs(got[t, h].astype(np.float64) - want)
+            err = np.abs(got[t, h] - want)
             assert (err <= bar).all(), (t, h, (err - bar).max())
