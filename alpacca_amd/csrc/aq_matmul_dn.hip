@@ -26,7 +26,7 @@
 //
 // 4096 x 4096 at M = 512 on the fp32 matrix cores (16x16x4 products at 1/16 of
 // the rate) and here: F16 248 -> 50 us a call, BF16 247 -> 63, F32 244 -> 114,
-// error against float64 8.1e-7 -> 4.1e-7, 6.9e-7 and 7.1e-7.  The fp32 kernel's
+// error against float64 8.1e-7 -> 2.9e-7, 6.9e-7 and 7.1e-7.  The fp32 kernel's
 // 128-row tiles also left small batches on few workgroups: 5414 x 12800 at M =
 // 2 F16 1198 -> 38 us (the weights alone: 29), F32 1311 -> 71.  What bounds it:
 // a stage's products and fragment reads (0.5 us of matrix cores in the 1.0 -

@@ -429,6 +429,9 @@ __global__ void __launch_bounds__(512)
 // constants are a fit to 4,028 timed calls (Q4_K, Q6_K, Q8_0, Q5_0; N 512 -
 // 14336, K 2048 - 14336, M 5 - 1500, every shape with up to eight splits): the
 // call they pick is 0.5 % slower than the fastest on average, 10 % at worst.
+// Q5_K goes by Q4_K's: 128 x 256 is its fastest too where they choose it (14336 x
+// 4096 at M = 512 131 us against 150 with 128 x 128, M = 2048 514 / 549), its worst
+// picks 12 - 13 % (M = 768 251 / 225, unsplit M = 128 59.9 / 52.8).
 constexpr TileCost kTiles[] = {
     {128, 256, {1.86f, 0.f, 0.f}, {0.f, 0.f, 0.f}, 3.6f},
     {128, 128, {1.15f, 1.55f, 1.33f}, {0.f, 0.f, 0.f}, 1.2f},

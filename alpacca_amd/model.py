@@ -195,7 +195,7 @@ class Model:
         self.n_past = 0
         self.cached_ids: list[int] = []
         # batched prefill: chunk size (ALPACCA_PREFILL_CHUNK, model.py:630-634)
-        # and matmul precision (fp32 MFMA: the reference's f32 products).  The
+        # and matmul precision (fp32: the reference's f32 products).  The
         # reference's 256 bounds host memory; here the chunk only sets how
         # many rows each matmul_t launch gets (the results are bit-identical
         # for every chunk size: a product's K order does not depend on M and
@@ -414,8 +414,8 @@ class Model:
 
     def _enqueue_prefill(self, tokens: list[int]) -> None:
         """The batched step over chunks of prefill_chunk tokens at positions
-        n_past..: RMSNorm of all rows, matmul_t for every projection (fp32
-        MFMA unless prefill_precision says otherwise), RoPE + KV store of the
+        n_past..: RMSNorm of all rows, matmul_t for every projection (float32
+        accuracy unless prefill_precision says otherwise), RoPE + KV store of the
         chunk, causal attention of its queries, SwiGLU, residual adds; then
         the head on the last token only, whose logits the stream leaves in
         self.logits."""
@@ -515,8 +515,9 @@ class Model:
         each, and where there are at least four times steps_per_graph of
         them, from twice steps_per_graph on, steps_per_graph steps each (the
         state advances on the device, so the steps are identical):
-        1807-1815 tok/s on the 1B model at 8-64 steps per graph against
-        1791-1793 at one.  `timing`, if given, receives the elapsed milliseconds of those n_gen - 1 decode steps
+        1830-1839 tok/s on the 1B model at 16 steps per graph against
+        1812-1826 at one (256 tokens after 2048).  `timing`, if given,
+        receives the elapsed milliseconds of those n_gen - 1 decode steps
         (HIP events on the launch stream), their count, and the wall time of
         the prompt (prefill_ms).
 
