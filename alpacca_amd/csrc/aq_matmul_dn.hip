@@ -87,7 +87,8 @@ __device__ __forceinline__ float bf16_finite(float x) {
 //   Else the pieces are bf16, e is 0 and the mark of rows with an infinity, a NaN
 //     or a value below kPieceMin other than zero kAgain.
 // Marked rows are corrected, or formed again, after the stores.
-// the smallest magnitude whose 24 bits three bf16 pieces hold: its last bit is
+
+// The smallest magnitude whose 24 bits three bf16 pieces hold: its last bit is
 // bf16's smallest subnormal, 2^-133 (the matrix cores keep subnormal inputs)
 constexpr float kPieceMin = 0x1p-110f;
 constexpr int kLoExp = 12, kList = 8, kAgain = 15;
@@ -297,7 +298,8 @@ template <int KIND, int MT, int NT, int WGM, int WGN, bool BARE>
 __global__ void __launch_bounds__(64 * WGM * WGN)
     k_mm_dn(const uint8_t *W, int64_t N, int64_t K, const uint16_t *xp, int64_t plane, int64_t Kp,
             const int32_t *__restrict__ xe, const Lacking *__restrict__ xl,
-            const float *__restrict__ X, int64_t M, float *__restrict__ Y, int per_split, int m_tiles, int n_tiles) {
+            const float *__restrict__ X, int64_t M, float *__restrict__ Y, int per_split, int m_tiles,
+            int n_tiles) {
   using T = DnTile<KIND, MT, NT, WGM, WGN>;
   constexpr int BM = T::BM, BN = T::BN, WAVES = T::kWaves, NX = pieces_of(KIND);
   constexpr int NB = KIND == kF32 ? 3 : 1;           // pieces of W
